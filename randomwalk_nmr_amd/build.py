@@ -18,8 +18,10 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["walk_kernels.hip", "zwalk_kernels.hip", "batch_kernels.hip", "backward_kernels.hip",
-               "locality_kernels.hip", "capi.hip", "drivers.hip", "probe_kernels.hip"]
+# the slowest to compile first
+HIP_SOURCES = ["zwalk_cpmg.hip", "zwalk_labels.hip", "zwalk_map.hip", "zwalk_kernels.hip", "zwalk_spec.hip",
+               "batch_kernels.hip", "walk_kernels.hip", "backward_kernels.hip", "locality_kernels.hip", "capi.hip",
+               "drivers.hip", "probe_kernels.hip"]
 CXX_SOURCES = ["laplace.cpp", "host_sim.cpp", "image_io.cpp", "histogram.cpp", "config.cpp", "output.cpp"]
 # the command-line program, linked against the library
 APP_SOURCE = "rwnmr_app.cpp"

@@ -1,6 +1,6 @@
-// zwalk_kernels.hip -- gfx950 CPMG / map walk for periodic and mirror
-// boundaries on the unfolded image (step described in zwalk_device.h), the
-// unfolded-image build and the Z-order sort keys.
+// zwalk_kernels.hip -- PFGSE on the unfolded image (step described in
+// zwalk_device.h), the unfolded-image build, the Z-order sort keys, and the
+// dispatch of the walks over their energy modes.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -11,133 +11,9 @@
 
 namespace rwnmr {
 
-template <int EMODE, int K, bool WRAPFIX, int CACHE, int TAB, bool NOFLUX = false, bool MFLAGS = false,
-          bool ADISP = false, bool HITS = true>
-__global__ __launch_bounds__(max_threads_for_k(K)) void zwalk_kernel(const WalkArgs a)
-{
-    __shared__ double lds[kEchoChunk][kEchoCols];
-    __shared__ uint4 tab[TAB == 1 ? kZWideEntries
-                                  : (TAB == 3 ? kZFlippedEntries : (MFLAGS ? 8 * kZFlagStride / 16 : (NOFLUX ? 12 : 6)))];
-    __shared__ uint4 small[6];
-    __shared__ uint2 fix[TAB == 3 ? kZFlippedEntries : (MFLAGS ? 8 * kZFlagStride / 16 : 6)];
-    __shared__ uint32_t keys[TAB == 3 ? kZFlagKeyEntries / 4 : (TAB == 2 ? kZKeyEntries / 4 : 1)];
-    __shared__ double ldelta[kMaxLabels];
-    extern __shared__ uint32_t zlh[];   // EMODE 2, K == 1: per-label hit counts (blockDim x kLhStride)
-    const uint64_t tile = tile_of_block(a);
-    if (a.tile_map && tile >= a.n_tiles)
-        return;  // spare workgroup of the XCD-striped grid (whole block leaves together)
-    uint8_t *key_bytes = reinterpret_cast<uint8_t *>(keys);
-    if (NOFLUX)
-        zbuild_table_noflux(a.zl, tab);
-    else if (TAB == 3)
-        zbuild_table_flipped(a.zl, tab, fix);
-    else if (MFLAGS)
-        zbuild_table_flags(a.zl, tab, fix);
-    else
-        zbuild_table(a.zl, TAB == 1 ? small : tab, fix);
-    if (TAB == 3)
-        zbuild_flag_key_table(keys);
-    if (TAB == 2)
-        zbuild_key_table(key_bytes, NOFLUX ? 32u : 16u);
-    if (EMODE == 2 && threadIdx.x < kMaxLabels)
-        ldelta[threadIdx.x] = (int)threadIdx.x < a.n_labels ? a.label_delta[threadIdx.x] : 1.0;
-    __syncthreads();
-    if (TAB == 1) {
-        zbuild_table_wide(small, tab);
-        __syncthreads();
-    }
-    zwalk_tile<EMODE, K, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, 1, false, ADISP, HITS>(
-        a, tile, a.partials ? a.partials + tile : nullptr, a.partial_stride, lds, tab, fix, ldelta, key_bytes,
-        EMODE == 2 && K == 1 ? zlh : nullptr);
-}
-
-// Speculative CPMG walk (zwalk_tile_spec): one walker per lane, for runs
-// too small to hide the chunk-load latency of a step.
-template <bool WRAPFIX, bool NOFLUX, bool MFLAGS>
-__global__ __launch_bounds__(1024) void zwalk_spec_kernel(const WalkArgs a)
-{
-    __shared__ double lds[kEchoChunk][kEchoCols];
-    __shared__ uint4 tab[MFLAGS ? 8 * kZFlagStride / 16 : (NOFLUX ? 12 : 6)];
-    __shared__ uint2 fix[MFLAGS ? 8 * kZFlagStride / 16 : 6];
-    __shared__ uint8_t keys[kZKeyEntries];
-    const uint64_t tile = tile_of_block(a);
-    if (a.tile_map && tile >= a.n_tiles)
-        return;  // spare workgroup of the XCD-striped grid (whole block leaves together)
-    if (NOFLUX)
-        zbuild_table_noflux(a.zl, tab);
-    else if (MFLAGS)
-        zbuild_table_flags(a.zl, tab, fix);
-    else
-        zbuild_table(a.zl, tab, fix);
-    zbuild_key_table(keys, NOFLUX ? 32u : 16u);
-    __syncthreads();
-    zwalk_tile_spec<WRAPFIX, NOFLUX, MFLAGS>(a, tile, a.partials ? a.partials + tile : nullptr, a.partial_stride,
-                                             lds, tab, fix, keys);
-}
-
-// Label-set CPMG: 8 sets of label deltas evaluated on one trajectory (one
-// walker per lane; zwalk_tile with NS = 8).  Unused sets (a.n_label_sets <
-// 8) carry deltas of 1.
-template <bool WRAPFIX, bool NOFLUX, bool MFLAGS>
-__global__ __launch_bounds__(1024) void zwalk_sets_kernel(const WalkArgs a)
-{
-    extern __shared__ double lds8[];   // kEchoChunk x 8 sets x waves of the block
-    __shared__ uint4 tab[MFLAGS ? 8 * kZFlagStride / 16 : (NOFLUX ? 12 : 6)];
-    __shared__ uint2 fix[MFLAGS ? 8 * kZFlagStride / 16 : 6];
-    __shared__ uint8_t keys[kZKeyEntries];
-    __shared__ double ldelta[8 * kMaxLabels];
-    const uint64_t tile = tile_of_block(a);
-    if (a.tile_map && tile >= a.n_tiles)
-        return;
-    if (NOFLUX)
-        zbuild_table_noflux(a.zl, tab);
-    else if (MFLAGS)
-        zbuild_table_flags(a.zl, tab, fix);
-    else
-        zbuild_table(a.zl, tab, fix);
-    zbuild_key_table(keys, NOFLUX ? 32u : 16u);
-    for (uint32_t t = threadIdx.x; t < 8u * kMaxLabels; t += blockDim.x) {
-        const uint32_t q = t / kMaxLabels, l = t % kMaxLabels;
-        ldelta[t] = (q < a.n_label_sets && (int)l < a.n_labels) ? a.label_delta[q * (uint32_t)a.n_labels + l] : 1.0;
-    }
-    __syncthreads();
-    zwalk_tile<2, 1, WRAPFIX, 128, 2, NOFLUX, MFLAGS, 8>(a, tile, a.partials ? a.partials + tile : nullptr,
-                                                         a.partial_stride, nullptr, tab, fix, ldelta, keys, nullptr,
-                                                         lds8);
-}
-
-// Jacobian forward: the per-label CPMG walk (zwalk_tile EMODE 2, one walker
-// per lane, per-label hit counts in LDS) that also sums h_l E per label and
-// echo (zwalk_tile JAC).  Dynamic LDS: the 8-label echo staging (kEchoChunk
-// x 8 x waves doubles), then the hit-count rows (blockDim x kLhStride).
-template <bool WRAPFIX, bool NOFLUX, bool MFLAGS>
-__global__ __launch_bounds__(1024) void zwalk_jac_kernel(const WalkArgs a)
-{
-    extern __shared__ double zjdyn[];
-    __shared__ double lds[kEchoChunk][kEchoCols];
-    __shared__ uint4 tab[MFLAGS ? 8 * kZFlagStride / 16 : (NOFLUX ? 12 : 6)];
-    __shared__ uint2 fix[MFLAGS ? 8 * kZFlagStride / 16 : 6];
-    __shared__ uint8_t keys[kZKeyEntries];
-    __shared__ double ldelta[kMaxLabels];
-    const uint64_t tile = tile_of_block(a);
-    if (a.tile_map && tile >= a.n_tiles)
-        return;
-    double *lds8 = zjdyn;
-    uint32_t *zlh = reinterpret_cast<uint32_t *>(zjdyn + (size_t)kEchoChunk * 8 * (blockDim.x / kWave));
-    if (NOFLUX)
-        zbuild_table_noflux(a.zl, tab);
-    else if (MFLAGS)
-        zbuild_table_flags(a.zl, tab, fix);
-    else
-        zbuild_table(a.zl, tab, fix);
-    zbuild_key_table(keys, NOFLUX ? 32u : 16u);
-    if (threadIdx.x < kMaxLabels)
-        ldelta[threadIdx.x] = (int)threadIdx.x < a.n_labels ? a.label_delta[threadIdx.x] : 1.0;
-    __syncthreads();
-    zwalk_tile<2, 1, WRAPFIX, 128, 2, NOFLUX, MFLAGS, 1, true>(a, tile, a.partials ? a.partials + tile : nullptr,
-                                                               a.partial_stride, lds, tab, fix, ldelta, keys, zlh,
-                                                               lds8);
-}
+// instantiated in zwalk_map.hip, zwalk_cpmg.hip and zwalk_labels.hip
+template <int EMODE>
+hipError_t launch_z_mode(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st);
 
 // PFGSE on the unfolded image: the walk between diffusion times counts hits
 // (register chunk cache, packed displacement flushed every kZFlush steps and
@@ -442,164 +318,6 @@ hipError_t launch_zkeys(const int32_t *x, const int32_t *y, const int32_t *z, ui
         return hipSuccess;
     hipLaunchKernelGGL(zkeys_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, x, y, z, n, zl, mflags, keys,
                        iota);
-    return hipGetLastError();
-}
-
-template <int EMODE, bool WRAPFIX, int CACHE, int TAB, bool NOFLUX = false, bool MFLAGS = false>
-static hipError_t launch_z(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
-{
-    // mirror CPMG of one walker per lane on images whose periods all exceed
-    // twice the flush interval: unbounded moves from address displacements
-    if constexpr (EMODE == 1 && MFLAGS && TAB == 3 && !NOFLUX) {
-        if (ls.k == 1 && zaddress_displacement_ok(a.zl)) {
-            // hit counts only when the caller asked for them
-            if (a.hits)
-                hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, true>), dim3(blocks),
-                                   dim3(ls.threads), 0, st, a);
-            else
-                hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, true, false>),
-                                   dim3(blocks), dim3(ls.threads), 0, st, a);
-            return hipGetLastError();
-        }
-    }
-    // EMODE 2 with one walker per lane keeps the per-label hit counts in LDS
-    const size_t lh_bytes = EMODE == 2 ? (size_t)kLhStride * ls.threads * sizeof(uint32_t) : 0;
-    switch (ls.k) {
-    case 1: hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS>), dim3(blocks), dim3(ls.threads), lh_bytes, st, a); break;
-    case 2: hipLaunchKernelGGL((zwalk_kernel<EMODE, 2, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS>), dim3(blocks), dim3(ls.threads), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((zwalk_kernel<EMODE, 4, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS>), dim3(blocks), dim3(ls.threads), 0, st, a); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-// a.zcache: 0 no chunk cache; 1 128-bit chunk with word select; 2 and 3 a
-// 128-bit chunk with the shift test and the direction drawn one step ahead,
-// through the byte-key table (2) or, for power-of-two periods, the wide
-// direction table (3; the 6-entry table otherwise); 4 the speculative CPMG
-// walk; 5 as 2 with a 64-bit (4 x 4 x 4 voxel) chunk, mirror walks with
-// reflection flags (others run 2).
-template <bool WRAPFIX, bool NOFLUX, bool MFLAGS>
-static hipError_t launch_z_spec(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
-{
-    hipLaunchKernelGGL((zwalk_spec_kernel<WRAPFIX, NOFLUX, MFLAGS>), dim3(blocks), dim3(ls.threads), 0, st, a);
-    return hipGetLastError();
-}
-
-template <int EMODE>
-static hipError_t launch_z_mode(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
-{
-    // a.zcache 4: the speculative CPMG walk (one walker per lane); other
-    // modes and lane shapes take the pipelined chunk-cache walk
-    if (a.zcache == 4 && EMODE == 1 && ls.k == 1) {
-        if (a.znoflux)
-            return launch_z_spec<false, true, false>(a, ls, blocks, st);
-        if (a.zmflags)
-            return a.zl.wrapfix ? launch_z_spec<true, false, true>(a, ls, blocks, st)
-                                : launch_z_spec<false, false, true>(a, ls, blocks, st);
-        return a.zl.wrapfix ? launch_z_spec<true, false, false>(a, ls, blocks, st)
-                            : launch_z_spec<false, false, false>(a, ls, blocks, st);
-    }
-    if (a.zcache == 4) {
-        WalkArgs b = a;
-        b.zcache = 2;
-        return launch_z_mode<EMODE>(b, ls, blocks, st);
-    }
-    if (a.znoflux)   // noflux on the periodic image: pipelined byte-key walk only
-        return a.zcache >= 2 ? launch_z<EMODE, false, 128, 2, true>(a, ls, blocks, st) : hipErrorInvalidValue;
-    if (a.zmflags && a.zcache == 5) {   // mirror, 8-byte chunk cache
-        if (EMODE < 2 && ls.threads >= 1024)
-            return a.zl.wrapfix ? launch_z<EMODE, true, 64, 3, false, true>(a, ls, blocks, st)
-                                : launch_z<EMODE, false, 64, 3, false, true>(a, ls, blocks, st);
-        return a.zl.wrapfix ? launch_z<EMODE, true, 64, 2, false, true>(a, ls, blocks, st)
-                            : launch_z<EMODE, false, 64, 2, false, true>(a, ls, blocks, st);
-    }
-    if (a.zcache == 5) {
-        WalkArgs b = a;
-        b.zcache = 2;
-        return launch_z_mode<EMODE>(b, ls, blocks, st);
-    }
-    if (a.zmflags && a.zcache >= 2) {   // mirror, walkers folded to the first octant with reflection flags
-        // CPMG and map walks of 1024-thread blocks read the flag-keyed
-        // tables (58 KiB of LDS: two blocks per CU, 8 waves per SIMD)
-        if (EMODE < 2 && ls.threads >= 1024)
-            return a.zl.wrapfix ? launch_z<EMODE, true, 128, 3, false, true>(a, ls, blocks, st)
-                                : launch_z<EMODE, false, 128, 3, false, true>(a, ls, blocks, st);
-        return a.zl.wrapfix ? launch_z<EMODE, true, 128, 2, false, true>(a, ls, blocks, st)
-                            : launch_z<EMODE, false, 128, 2, false, true>(a, ls, blocks, st);
-    }
-    if (a.zl.wrapfix) {
-        switch (a.zcache) {
-        case 0: return launch_z<EMODE, true, 0, 0>(a, ls, blocks, st);
-        case 1: return launch_z<EMODE, true, 1, 0>(a, ls, blocks, st);
-        case 2: return launch_z<EMODE, true, 128, 2>(a, ls, blocks, st);
-        case 3: return launch_z<EMODE, true, 128, 0>(a, ls, blocks, st);
-        default: return hipErrorInvalidValue;
-        }
-    }
-    switch (a.zcache) {
-    case 0: return launch_z<EMODE, false, 0, 0>(a, ls, blocks, st);
-    case 1: return launch_z<EMODE, false, 1, 0>(a, ls, blocks, st);
-    case 2: return launch_z<EMODE, false, 128, 2>(a, ls, blocks, st);
-    case 3: return launch_z<EMODE, false, 128, 1>(a, ls, blocks, st);
-    default: return hipErrorInvalidValue;
-    }
-}
-
-hipError_t launch_zwalk_sets(const WalkArgs &a, uint32_t threads, hipStream_t st)
-{
-    if (a.n == 0)
-        return hipSuccess;
-    if (a.shift != 0 || !a.zwords || !a.zlabels || !a.label_delta || a.n_labels <= 0 || a.n_labels > kMaxLabels ||
-        a.n_label_sets == 0 || a.n_label_sets > 8 || threads == 0 || threads > 1024 || threads % 64 != 0)
-        return hipErrorInvalidValue;
-    const uint64_t tiles = (a.n + threads - 1) / threads;
-    if (tiles > 0x7FFFFFF0ull || (a.tile_map && a.n_tiles != tiles))
-        return hipErrorInvalidValue;
-    const uint32_t blocks = a.tile_map ? (uint32_t)(((tiles + kXcds - 1) / kXcds) * kXcds) : (uint32_t)tiles;
-    // the per-set echo staging, sized for this block's waves
-    const size_t lds8_bytes = (size_t)kEchoChunk * 8 * (threads / kWave) * sizeof(double);
-    if (a.znoflux) {
-        hipLaunchKernelGGL((zwalk_sets_kernel<false, true, false>), dim3(blocks), dim3(threads), lds8_bytes, st, a);
-    } else if (a.zmflags) {
-        if (a.zl.wrapfix)
-            hipLaunchKernelGGL((zwalk_sets_kernel<true, false, true>), dim3(blocks), dim3(threads), lds8_bytes, st, a);
-        else
-            hipLaunchKernelGGL((zwalk_sets_kernel<false, false, true>), dim3(blocks), dim3(threads), lds8_bytes, st,
-                               a);
-    } else if (a.zl.wrapfix) {
-        hipLaunchKernelGGL((zwalk_sets_kernel<true, false, false>), dim3(blocks), dim3(threads), lds8_bytes, st, a);
-    } else {
-        hipLaunchKernelGGL((zwalk_sets_kernel<false, false, false>), dim3(blocks), dim3(threads), lds8_bytes, st, a);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_zwalk_jac(const WalkArgs &a, uint32_t threads, hipStream_t st)
-{
-    if (a.n == 0)
-        return hipSuccess;
-    if (a.shift != 0 || !a.zwords || !a.zlabels || !a.label_delta || !a.partials || !a.jac_partials ||
-        a.n_labels <= 0 || a.n_labels > kMaxLabels || threads == 0 || threads > 1024 || threads % 64 != 0)
-        return hipErrorInvalidValue;
-    const uint64_t tiles = (a.n + threads - 1) / threads;
-    if (tiles > 0x7FFFFFF0ull || (a.tile_map && a.n_tiles != tiles))
-        return hipErrorInvalidValue;
-    const uint32_t blocks = a.tile_map ? (uint32_t)(((tiles + kXcds - 1) / kXcds) * kXcds) : (uint32_t)tiles;
-    const size_t dyn = (size_t)kEchoChunk * 8 * (threads / kWave) * sizeof(double) +
-                       (size_t)kLhStride * threads * sizeof(uint32_t);
-    if (a.znoflux) {
-        hipLaunchKernelGGL((zwalk_jac_kernel<false, true, false>), dim3(blocks), dim3(threads), dyn, st, a);
-    } else if (a.zmflags) {
-        if (a.zl.wrapfix)
-            hipLaunchKernelGGL((zwalk_jac_kernel<true, false, true>), dim3(blocks), dim3(threads), dyn, st, a);
-        else
-            hipLaunchKernelGGL((zwalk_jac_kernel<false, false, true>), dim3(blocks), dim3(threads), dyn, st, a);
-    } else if (a.zl.wrapfix) {
-        hipLaunchKernelGGL((zwalk_jac_kernel<true, false, false>), dim3(blocks), dim3(threads), dyn, st, a);
-    } else {
-        hipLaunchKernelGGL((zwalk_jac_kernel<false, false, false>), dim3(blocks), dim3(threads), dyn, st, a);
-    }
     return hipGetLastError();
 }
 
