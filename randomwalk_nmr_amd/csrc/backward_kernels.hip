@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kZBackThreads) void zbackward_kernel(const WalkArgs
     __shared__ double lds[kMaxLabels][kMaxWaves];
     __shared__ uint4 tab[6];
     __shared__ uint2 fix[6];
-    __shared__ uint8_t keys[kZKeyEntries];
+    __shared__ __align__(16) uint8_t keys[kZKeyEntries];
     __shared__ double ldelta[kMaxLabels];
     // R_wl, label-major: the block size is fixed, so a label's offset is one
     // shift-and-add, and 32 KiB keeps 4 blocks (8 waves per SIMD) per CU
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(kZBackThreads) void zbackward_kernel(const WalkArgs
     double Q = 0.0;
     uint32_t QB = 0xFFFFFFFFu;
     uint4 QV = make_uint4(0u, 0u, 0u, 0u);
-    const zrsrc_t zrsrc = zchunk_rsrc(a.zwords, a.zl);
+    const zrsrc_t zrsrc = zchunk_rsrc(a.zwords, a.zl.bits);
     const char *tab_bytes = reinterpret_cast<const char *>(tab);
     const char *fix_bytes = reinterpret_cast<const char *>(fix);
     ZEntry T;
@@ -170,11 +170,11 @@ __global__ __launch_bounds__(kZBackThreads) void zbackward_kernel(const WalkArgs
         // overlaps the chunk load's
         __builtin_amdgcn_sched_barrier(0);
         settle();
-        if (__builtin_expect(zchunk_wall<128>(c, QV) != 0u, 0)) {
+        const uint32_t wall = zchunk_wall<128>(c, QV);
+        A = zsel(wall, A, c);
+        if (__builtin_expect(wall != 0u, 0)) {
             lab = zlabel_at(a, c);
             pend = true;
-        } else {
-            A = c;
         }
     };
     const uint32_t e0 = seg * b.every;

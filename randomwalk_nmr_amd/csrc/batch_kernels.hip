@@ -27,7 +27,7 @@ __global__ __launch_bounds__(256) void batch_kernel(const BatchArgs b)
     __shared__ double lds[kEchoChunk][kEchoCols];
     __shared__ uint4 tab[6];
     __shared__ uint2 fix[6];
-    __shared__ uint8_t keys[kZKeyEntries];   // the byte-key table: the same for every instance
+    __shared__ __align__(16) uint8_t keys[kZKeyEntries];   // the byte-key table: the same for every instance
     __shared__ uint32_t next;
     zbuild_key_table(keys);
     for (;;) {

@@ -109,6 +109,8 @@ struct rwnmr_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     LaunchShape shape{256, 1};
+    // no shape / no image form was asked for: run_shape and attach_zimage choose by the run
+    bool shape_auto = true, form_auto = true;
     // walker staging for host-pointer calls
     DevBuf x, y, z, seed, energy, hits, penalty, x0, y0, z0;
     // per-call small arrays and reductions
@@ -152,8 +154,8 @@ struct rwnmr_ctx {
     // chunk cache, 3 and 4 with the chunk tested by one shift and the next
     // direction drawn a step ahead, through the 4 KiB byte-key table (3, the
     // default) or the 64 KiB wide direction table (4); 5 the speculative
-    // CPMG walk; 6 as 3 with an 8-byte (4 x 4 x 4 voxel) chunk for mirror
-    // walks (others run 3)
+    // CPMG and map walk; 6 as 3 with an 8-byte (4 x 4 x 4 voxel) chunk for
+    // mirror walks (others run 3)
     int unfolded = 3;
     // resident 1024-thread blocks of the flag-keyed mirror walk (two per CU):
     // the tile count of balanced tiles (zbalanced_tile_walkers)
@@ -487,6 +489,13 @@ const uint8_t *zlabels_for(rwnmr_ctx *c, const rwnmr_image *img, int bc)
     return z.lstate == 1 ? z.labels : nullptr;
 }
 
+// Walker counts up to one wave per SIMD (1024 SIMDs x 64 lanes) take the
+// speculative walk (form 5), with its two loads per step: 139 against 203 ns
+// per step of 10k walkers at 128^3 (mirror), 167 against 197 at 65,536, but
+// 245 against 222 at 100k and 545 against 297 at 200k, where the loads of
+// several waves per SIMD queue up.  The autotuner times it up to here too.
+constexpr uint64_t kSpecMaxWalkers = 1024ull * 64ull;
+
 // Use the unfolded-image kernel for this walk when one applies.  noflux_ok:
 // the caller's kernel also runs noflux walks on the periodic unfolded image
 // (the CPMG, map and PFGSE walks, with the pipelined forms 3 and 4 and every
@@ -505,8 +514,19 @@ void attach_zimage(rwnmr_ctx *c, const rwnmr_image *img, int bc, int emode, Walk
     rwnmr::zoctant_constants(a, false);
     a.znoflux = 0;
     a.zmflags = 0;
-    if (emode < 0 || emode > 2 || a.shift != 0)
+    if (emode < 0 || emode > 2)
         return;
+    const uint32_t f = bc == rwnmr::kMirror ? 2u : 1u;
+    rwnmr::ZLayout sub{};
+    if (a.shift != 0) {
+        // voxel division: sub-voxel addresses (3 bits per voxel level more)
+        // must fit 32 bits, else the folded kernel walks
+        const uint64_t side = (uint64_t)std::max(img->W, std::max(img->H, img->D));
+        if (c->unfolded < 3 || a.shift > 10 || ((f * side) << a.shift) > 0x7FFFFFFFull ||
+            !rwnmr::zlayout_make((f * (uint32_t)img->W) << a.shift, (f * (uint32_t)img->H) << a.shift,
+                                 (f * (uint32_t)img->D) << a.shift, sub))
+            return;
+    }
     int zbc = bc;
     if (bc == rwnmr::kNoflux) {
         if (!noflux_ok || c->unfolded < 3 || img->W < 2 || img->H < 2 || img->D < 2)
@@ -520,13 +540,30 @@ void attach_zimage(rwnmr_ctx *c, const rwnmr_image *img, int bc, int emode, Walk
         a.zwords = z->words;
         a.zl = z->zl;
         a.zcache = c->unfolded >= 2 ? (uint32_t)(c->unfolded - 1) : 0u;
+        // few walkers: the speculative walk, unless a form or a shape was asked for
+        if (c->form_auto && c->shape_auto && emode < 2 && a.n <= kSpecMaxWalkers)
+            a.zcache = 4;
         a.zlabels = zlab;
         // mirror image of equal power-of-two periods: labels kept for the
         // first octant and read at the folded address
         rwnmr::zoctant_constants(a, zlab && bc == rwnmr::kMirror && rwnmr::zoctant_layout(z->zl));
+        if (a.shift != 0)
+            a.zl = sub;
         a.znoflux = bc == rwnmr::kNoflux ? 1u : 0u;
         a.zmflags = (bc == rwnmr::kMirror && mflags_ok && c->unfolded >= 3) ? 1u : 0u;
     }
+}
+
+// Launch shape of a CPMG or map run (a as attach_zimage left it): the
+// context's, or, where none was set, 64-thread blocks for a speculative walk
+// that leaves a SIMD of each CU free, so that its waves spread over as many
+// CUs as there are (128^3, 30k walkers: 152 ns per step against 176 with 256
+// threads; 65,536 walkers: 178 against 167).
+LaunchShape run_shape(const rwnmr_ctx *c, const WalkArgs &a, int emode)
+{
+    return c->shape_auto && a.zwords && a.zcache == 4 && emode < 2 && a.n <= kSpecMaxWalkers / 4 * 3
+               ? LaunchShape{64u, 1u}
+               : c->shape;
 }
 
 hipError_t launch_any_walk(const WalkArgs &a, int bc, int emode, const LaunchShape &ls, hipStream_t st)
@@ -557,9 +594,6 @@ bool k_rows_arithmetic(const double *k, uint64_t nkv, uint32_t n_k, uint32_t n_r
 // Upper bound on the partial-sum scratch of one walk launch; longer CPMG runs
 // are split into several launches of fewer echoes.
 constexpr uint64_t kMaxPartialBytes = 1ull << 30;
-// walker counts up to one wave per SIMD (1024 SIMDs x 64 lanes): the
-// autotuner also times the speculative walk (form 5) for these
-constexpr uint64_t kSpecMaxWalkers = 1024ull * 64ull;
 
 // Tiles (echo-partial columns) of a walk launch over a.n walkers: balanced
 // tiles (zbalanced_tile_walkers, which set a.tile_walkers) or the usual grid
@@ -581,12 +615,11 @@ uint32_t walk_columns(const rwnmr_ctx *c, WalkArgs &a, int emode, const LaunchSh
 // the unsorted walk; echo sums differ only by summation order.
 // `a` holds the caller's (or staged) device arrays; sums is device or null.
 rwnmr_status walk_local(rwnmr_ctx *c, const rwnmr_image *img, const WalkArgs &a, int bc, int emode, uint32_t echoes,
-                        uint32_t steps_per_echo, double *sums, uint64_t max_chunk)
+                        uint32_t steps_per_echo, double *sums, uint64_t max_chunk, const LaunchShape &ls)
 {
     const uint64_t n = a.n;
     if (n > 0xFFFFFFFFull)
         return fail(c, RWNMR_ERR_INVALID, "locality ordering supports up to 2^32 walkers");
-    const LaunchShape ls = c->shape;
     // a's tiles (balanced tiles when walk_columns set them)
     const uint64_t per_tile = a.tile_walkers ? (uint64_t)a.tile_walkers : (uint64_t)ls.threads * ls.k;
     const uint32_t tiles = (uint32_t)((n + per_tile - 1) / per_tile);
@@ -778,7 +811,7 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
     if (jac && (!a.zwords || !a.zlabels))
         return fail(c, RWNMR_ERR_INVALID, "Jacobian forward: needs the unfolded labelled image");
     // the Jacobian forward holds one walker per lane
-    const LaunchShape shape = jac ? LaunchShape{c->shape.threads, 1u} : c->shape;
+    const LaunchShape shape = jac ? LaunchShape{c->shape.threads, 1u} : run_shape(c, a, emode);
     // tiles, one echo-partial column each (balanced tiles where they apply)
     const uint32_t blocks = jac ? rwnmr::walk_grid_blocks(w->n, shape, (int)shift) : walk_columns(c, a, emode, shape);
     a.partial_stride = blocks;
@@ -815,8 +848,8 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
     const bool local = emode < 2 && shift == 0 && c->locality && w->n >= c->locality_min_walkers;
     if (local) {
         a.steps_per_echo = steps_per_echo;
-        if ((s = walk_local(c, img, a, bc, emode, echoes, steps_per_echo, echo_sums ? sums : nullptr, chunk)) !=
-            RWNMR_OK)
+        if ((s = walk_local(c, img, a, bc, emode, echoes, steps_per_echo, echo_sums ? sums : nullptr, chunk,
+                            shape)) != RWNMR_OK)
             return s;
     } else {
     if (a.energy == nullptr && chunk < echoes && w->n) {
@@ -845,7 +878,7 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
         if (jac)
             RW_HIP(c, rwnmr::launch_zwalk_jac(a, shape.threads, c->stream));
         else
-            RW_HIP(c, launch_any_walk(a, bc, emode, c->shape, c->stream));
+            RW_HIP(c, launch_any_walk(a, bc, emode, shape, c->stream));
         timing_end(c, t0);
         if (echo_sums) {
             // rows 0..ne of this launch are echoes done..done+ne (row 0 repeats
@@ -994,6 +1027,7 @@ rwnmr_status rwnmr_ctx_set_unfolded(rwnmr_ctx *c, int32_t enable)
     if (enable < 0 || enable > 6)
         return fail(c, RWNMR_ERR_INVALID, "set_unfolded: mode must be 0 .. 6");
     c->unfolded = enable;
+    c->form_auto = false;
     return RWNMR_OK;
 }
 
@@ -1035,6 +1069,7 @@ rwnmr_status rwnmr_ctx_set_launch(rwnmr_ctx *c, uint32_t tpb, uint32_t k)
 {
     if (!c)
         return RWNMR_ERR_INVALID;
+    const bool use_default = tpb == 0 && k == 0;
     if (tpb == 0)
         tpb = 256;
     if (k == 0)
@@ -1044,6 +1079,7 @@ rwnmr_status rwnmr_ctx_set_launch(rwnmr_ctx *c, uint32_t tpb, uint32_t k)
                     "threads_per_block must be a multiple of 64 and at most 1024 (k=1), 512 (k=2) or 256 (k=4)");
     c->shape.threads = tpb;
     c->shape.k = k;
+    c->shape_auto = use_default;
     return RWNMR_OK;
 }
 
@@ -1212,7 +1248,7 @@ rwnmr_status rwnmr_map_run(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *
         const uint32_t now = (uint32_t)std::min<uint64_t>(left, 1ull << 30);
         a.steps_per_echo = now;
         hipEvent_t t0 = timing_begin(c);
-        RW_HIP(c, launch_any_walk(a, bc, 0, c->shape, c->stream));
+        RW_HIP(c, launch_any_walk(a, bc, 0, run_shape(c, a, 0), c->stream));
         timing_end(c, t0);
         left -= now;
     }
@@ -1261,7 +1297,10 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
     const LaunchShape saved = c->shape;
     const int saved_unfolded = c->unfolded;
     const uint32_t saved_resort = c->resort_every;
+    const bool saved_form_auto = c->form_auto, saved_shape_auto = c->shape_auto;
     auto restore = [&]() {
+        c->form_auto = saved_form_auto;
+        c->shape_auto = saved_shape_auto;
         c->timing = was_timing;
         c->kernel_ms = saved_ms;
         c->kernel_launches = saved_launches;
@@ -1271,6 +1310,7 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
         cleanup();
     };
     c->timing = true;
+    c->form_auto = c->shape_auto = false;   // each trial runs the shape and form it is set to
     (void)hipStreamSynchronize(c->stream);
     timing_collect(c);
     // One trial run from the caller's start state; returns the walk kernels'
@@ -1483,7 +1523,13 @@ rwnmr_status rwnmr_cpmg_run_noalloc(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_
     uint32_t *flag = static_cast<uint32_t *>(c->scratch);
     double *part = reinterpret_cast<double *>(static_cast<unsigned char *>(c->scratch) + kScratchFlagBytes);
     const uint64_t part_doubles = (kScratchBytes - kScratchFlagBytes) / sizeof(double);
-    const uint32_t blocks = rwnmr::walk_grid_blocks(w->n, c->shape, (int)shift);
+    const WalkerView v{w->x, w->y, w->z, w->seed, w->energy, w->hits, w->penalty};
+    WalkArgs a = base_args(img, v, w, shift, flag);
+    a.n_labels = img->n_labels;
+    // an unfolded image is used only when an earlier call built it
+    attach_zimage(c, img, bc, 1, a, true, true, false);
+    const LaunchShape shape = run_shape(c, a, 1);
+    const uint32_t blocks = rwnmr::walk_grid_blocks(w->n, shape, (int)shift);
     // echoes per launch: rows 0..chunk of [echo][block] partials must fit the scratch
     uint64_t chunk = echoes ? echoes : 1;
     if (echo_sums && blocks) {
@@ -1505,11 +1551,6 @@ rwnmr_status rwnmr_cpmg_run_noalloc(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, c->stream, flag, 0u, 1ull);
     RW_HIP(c, hipGetLastError());
     c->scratch_flag_pending = true;
-    const WalkerView v{w->x, w->y, w->z, w->seed, w->energy, w->hits, w->penalty};
-    WalkArgs a = base_args(img, v, w, shift, flag);
-    a.n_labels = img->n_labels;
-    // an unfolded image is used only when an earlier call built it
-    attach_zimage(c, img, bc, 1, a, true, true, false);
     a.partial_stride = blocks;
     a.steps_per_echo = steps_per_echo;
     uint32_t done = 0;
@@ -1517,7 +1558,7 @@ rwnmr_status rwnmr_cpmg_run_noalloc(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_
         const uint32_t ne = (uint32_t)std::min<uint64_t>(chunk, (uint64_t)echoes - done);
         a.echoes = ne;
         a.partials = echo_sums ? part : nullptr;
-        RW_HIP(c, launch_any_walk(a, bc, 1, c->shape, c->stream));
+        RW_HIP(c, launch_any_walk(a, bc, 1, shape, c->stream));
         if (echo_sums)
             RW_HIP(c, rwnmr::launch_reduce_rows(part, (uint64_t)ne + 1, blocks, echo_sums + done, c->stream));
         done += ne;
@@ -1574,12 +1615,6 @@ rwnmr_status rwnmr_cpmg_graph_create(rwnmr_ctx *c, const rwnmr_image *img, rwnmr
         return fail(c, RWNMR_ERR_INVALID,
                     "cpmg_graph_create: device walkers, and start arrays (if given) of the same count on the device");
     const uint64_t n = w->n;
-    const uint32_t blocks = rwnmr::walk_grid_blocks(n, c->shape, 0);
-    uint64_t chunk = echoes ? echoes : 1;
-    if (echo_sums && blocks)
-        chunk = std::min<uint64_t>(chunk, std::max<uint64_t>(2, kMaxPartialBytes / (8ull * blocks)) - 1);
-    if (chunk < echoes && !w->energy && n)
-        return fail(c, RWNMR_ERR_INVALID, "cpmg_graph_create: a run of several launches needs a device energy array");
     // everything the graph touches exists before the capture: the error word,
     // the unfolded image and the graph's own partials
     RW_HIP(c, c->flag.reserve(sizeof(uint32_t)));
@@ -1587,6 +1622,13 @@ rwnmr_status rwnmr_cpmg_graph_create(rwnmr_ctx *c, const rwnmr_image *img, rwnmr
     WalkArgs a = base_args(img, v, w, 0, c->flag.as<uint32_t>());
     a.n_labels = img->n_labels;
     attach_zimage(c, img, bc, 1, a, true, true, true);
+    const LaunchShape shape = run_shape(c, a, 1);
+    const uint32_t blocks = rwnmr::walk_grid_blocks(n, shape, 0);
+    uint64_t chunk = echoes ? echoes : 1;
+    if (echo_sums && blocks)
+        chunk = std::min<uint64_t>(chunk, std::max<uint64_t>(2, kMaxPartialBytes / (8ull * blocks)) - 1);
+    if (chunk < echoes && !w->energy && n)
+        return fail(c, RWNMR_ERR_INVALID, "cpmg_graph_create: a run of several launches needs a device energy array");
     a.partial_stride = blocks;
     a.steps_per_echo = steps_per_echo;
     a.tile_map = 1;
@@ -1630,7 +1672,7 @@ rwnmr_status rwnmr_cpmg_graph_create(rwnmr_ctx *c, const rwnmr_image *img, rwnmr
             const uint32_t ne = (uint32_t)std::min<uint64_t>(chunk, (uint64_t)echoes - done);
             a.echoes = ne;
             a.partials = echo_sums ? g->partials : nullptr;
-            RW_HIP(c, launch_any_walk(a, bc, 1, c->shape, c->stream));
+            RW_HIP(c, launch_any_walk(a, bc, 1, shape, c->stream));
             if (echo_sums)
                 RW_HIP(c, rwnmr::launch_reduce_rows(g->partials, (uint64_t)ne + 1, blocks, echo_sums + done,
                                                     c->stream));

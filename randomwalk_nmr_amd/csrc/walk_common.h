@@ -177,9 +177,9 @@ RW_HD uint32_t morton3(uint32_t bx, uint32_t by, uint32_t bz)
 // axis is then three 32-bit operations on A (a dilated add):
 //     +1: A' = (A & ~M) | (((A | ~M) + lowbit(M)) & M)
 //     -1: A' = (A & ~M) | (((A | ~M) + M) & M)
-// both wrapping at 2^k.  A period that is not a power of two needs one fix
-// after the add (field == dep(P) -> 0 going up; field == all ones ->
-// dep(P - 1) going down).
+// both wrapping at 2^k.  A period P that is not a power of two wraps by a test
+// of the current address beside the add (field == dep(P - 1) going up: the new
+// field is 0; field == 0 going down: dep(P - 1)).
 // Bit order: each aligned run of 64 addresses is one 64-bit value (word
 // 2i the low half, 2i + 1 the high half) holding address a at bit
 // 63 - (a & 63), so a left shift by a & 63 (the hardware count of a 64-bit
@@ -269,24 +269,19 @@ struct ZDir {
     uint32_t add;     // lowbit(mask) going up, mask going down
     int32_t dp;       // packed unbounded displacement: +-1 (x), +-2^10 (y), +-2^20 (z)
     uint32_t m;       // mask of the moving axis
-    uint32_t wrapv;   // field value that needs the wrap fix (never matches if none)
-    uint32_t fixv;    // replacement field value
+    uint32_t wrapv;   // current field value that wraps (never matches if none)
+    uint32_t fixv;    // field value after the wrap
 };
 
 // Noflux move on the periodic unfolded image (period = image size, every
-// size >= 2): the forward move (m, add, dp) crosses the face when
-// ((c & mp) | (A & mm)) == tgt (c: the candidate, A: the current address;
-// going up the field wraps to 0 or, for a period that is not a power of
-// two, reaches the period; going down the walker is at 0); the reference
-// then turns around (B/NMR_Simulation/NMR_cpmg_cuda.cpp:1847-1902): addend
-// add2, displacement dp2.  Walkers never leave the image, so no wrap
-// fix-up is needed.
-struct ZFlip {
-    uint32_t m, add;
-    int32_t dp;
-    uint32_t tgt, add2;
-    int32_t dp2;
-    uint32_t mp, mm;
+// size >= 2): a walker in the last voxel of its axis (the first, going down)
+// turns around (B/NMR_Simulation/NMR_cpmg_cuda.cpp:1847-1902), so the move
+// adds add2 instead of add when (A & mf) == tgt, A the current address and
+// mf the address bits of the axis' voxel (of all the axis without voxel
+// division).  Walkers never leave the image, so no wrap is needed and their
+// coordinates are the address itself.
+struct ZFace {
+    uint32_t m, add, mf, tgt, add2;
 };
 
 // s % 6 residue for table index idx (inverse of the CRT pairing).
@@ -313,24 +308,27 @@ RW_HD uint32_t zdot4(uint32_t a, uint32_t w, uint32_t acc)
 
 RW_HD uint32_t zkey_index(uint32_t k) { return 2u * (k % 3u) + (k & 1u); }
 
-RW_HD ZFlip zdir_noflux(const ZLayout &L, uint32_t idx)
+// shift: log2 of the voxel division (the low 3 shift address bits are the
+// position inside the voxel).
+RW_HD ZFace zdir_face(const ZLayout &L, uint32_t idx, uint32_t shift = 0u)
 {
     const uint32_t r = zdir_residue(idx);
     const int ax = move_axis(r), sg = move_sign(r);
     const uint32_t m = L.m[ax], low = m & (~m + 1u);
-    const int32_t unit = ax == 0 ? 1 : (ax == 1 ? 1 << 10 : 1 << 20);
-    const uint32_t k = (uint32_t)__builtin_popcount(m);
-    const uint32_t p = L.period[ax];
-    ZFlip f;
+    ZFace f;
     f.m = m;
     f.add = sg > 0 ? low : m;
-    f.dp = sg * unit;
     f.add2 = sg > 0 ? m : low;
-    f.dp2 = -sg * unit;
-    f.mp = sg > 0 ? m : 0u;
-    f.mm = sg > 0 ? 0u : m;
-    f.tgt = (sg > 0 && (1ull << k) != (uint64_t)p) ? zdeposit(p, m) : 0u;
+    f.mf = m & ~((1u << (3u * shift)) - 1u);
+    f.tgt = sg > 0 ? (zdeposit(L.period[ax] - 1u, m) & f.mf) : 0u;
     return f;
+}
+
+// Candidate address of a noflux move.
+RW_HD uint32_t zmove_face(uint32_t A, const ZFace &f)
+{
+    const uint32_t add = (A & f.mf) == f.tgt ? f.add2 : f.add;
+    return (A & ~f.m) | (((A | ~f.m) + add) & f.m);
 }
 
 // flags: bit a reverses the address move along axis a (the mirror image of
@@ -354,10 +352,10 @@ RW_HD ZDir zdir_make(const ZLayout &L, uint32_t idx, uint32_t flags = 0u)
         d.wrapv = 0xFFFFFFFFu;   // no axis owns every bit, so this never matches
         d.fixv = 0;
     } else if (sg > 0) {
-        d.wrapv = zdeposit(p, m);
+        d.wrapv = zdeposit(p - 1u, m);
         d.fixv = 0;
     } else {
-        d.wrapv = m;
+        d.wrapv = 0;
         d.fixv = zdeposit(p - 1u, m);
     }
     return d;
@@ -366,10 +364,9 @@ RW_HD ZDir zdir_make(const ZLayout &L, uint32_t idx, uint32_t flags = 0u)
 // Candidate address after one move.
 RW_HD uint32_t zmove(uint32_t A, const ZDir &d, int wrapfix)
 {
-    uint32_t c = (A & d.nm) | (((A | d.nm) + d.add) & ~d.nm);
-    if (wrapfix && (c & d.m) == d.wrapv)
-        c = (c & d.nm) | d.fixv;
-    return c;
+    if (wrapfix && (A & d.m) == d.wrapv)
+        return (A & d.nm) | d.fixv;
+    return (A & d.nm) | (((A | d.nm) + d.add) & ~d.nm);
 }
 
 // Byte sum of the 64-bit state (== state mod 3, since 256 == 1 mod 3) and

@@ -32,6 +32,27 @@
 
 namespace rwnmr {
 
+// Bitwise select m ? a : b.  v_bitop3_b32 issues in 2 cycles per wave on
+// gfx950, v_bfi_b32 (which the compiler makes of the and-or form) in 4, a
+// compare and v_cndmask_b32 in 6, and more where several selects follow each
+// other; the walls and chunk halves of a step are therefore picked under sign
+// masks.
+__device__ __forceinline__ uint32_t zsel(uint32_t m, uint32_t a, uint32_t b)
+{
+    return __builtin_amdgcn_bitop3_b32(m, a, b, 0xCAu);
+}
+
+__device__ __forceinline__ uint64_t zsel64(uint32_t m, uint64_t a, uint64_t b)
+{
+    return ((uint64_t)zsel(m, (uint32_t)(a >> 32), (uint32_t)(b >> 32)) << 32) | zsel(m, (uint32_t)a, (uint32_t)b);
+}
+
+__device__ __forceinline__ double zsel_f64(uint32_t m, double a, double b)
+{
+    return __hiloint2double((int)zsel(m, (uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b)),
+                            (int)zsel(m, (uint32_t)__double2loint(a), (uint32_t)__double2loint(b)));
+}
+
 __device__ __forceinline__ uint32_t zaddress(int32_t x, int32_t y, int32_t z, const ZLayout &zl)
 {
     return zdeposit(floor_mod(x, zl.period[0]), zl.m[0]) | zdeposit(floor_mod(y, zl.period[1]), zl.m[1]) |
@@ -103,8 +124,24 @@ static_assert(kZKeyEntries > kZKeyMax && kZKeyEntries % 64u == 0u, "key table si
 // or 32 for the noflux table).
 __device__ __forceinline__ void zbuild_key_table(uint8_t *keys, uint32_t bytes = 16u)
 {
-    for (uint32_t e = threadIdx.x; e < kZKeyEntries; e += blockDim.x)
-        keys[e] = (uint8_t)(bytes * zkey_index(e));
+    // entries repeat every 6 keys, so words of 4 keys every 3 words and
+    // 16-byte groups every 3 groups: one wide store per 16 keys
+    uint32_t w[3];
+#pragma unroll
+    for (uint32_t i = 0; i < 3u; ++i) {
+        w[i] = 0u;
+#pragma unroll
+        for (uint32_t b = 0; b < 4u; ++b)
+            w[i] |= (bytes * zkey_index(4u * i + b)) << (8u * b);
+    }
+    uint4 *out = reinterpret_cast<uint4 *>(keys);
+    for (uint32_t g = threadIdx.x; g < kZKeyEntries / 16u; g += blockDim.x) {
+        const uint32_t r = g % 3u;   // group g starts at word 4 g = g (mod 3)
+        const uint32_t w0 = r == 0u ? w[0] : (r == 1u ? w[1] : w[2]);
+        const uint32_t w1 = r == 0u ? w[1] : (r == 1u ? w[2] : w[0]);
+        const uint32_t w2 = r == 0u ? w[2] : (r == 1u ? w[0] : w[1]);
+        out[g] = make_uint4(w0, w1, w2, w0);
+    }
 }
 
 // Flag-keyed byte tables (TAB 3; mirror walks with reflection flags): the
@@ -151,15 +188,15 @@ __device__ __forceinline__ void zbuild_flag_key_table(uint32_t *keys)
     }
 }
 
-// Noflux direction table of layout zl (periodic image): two 16-byte halves
-// per direction, {m, add, dp, tgt} and {add2, dp2, mp, mm} (ZFlip).
-// Threads 0..5 write; the caller syncs.
-__device__ __forceinline__ void zbuild_table_noflux(const ZLayout &zl, uint4 *tab)
+// Noflux direction table of layout zl (periodic image, sub-voxel addresses
+// with a voxel division of 2^shift): two 16-byte halves per direction, {m,
+// add, mf, tgt} and {add2} (ZFace).  Threads 0..5 write; the caller syncs.
+__device__ __forceinline__ void zbuild_table_noflux(const ZLayout &zl, uint4 *tab, uint32_t shift = 0u)
 {
     if (threadIdx.x < 6) {
-        const ZFlip f = zdir_noflux(zl, threadIdx.x);
-        tab[2 * threadIdx.x] = make_uint4(f.m, f.add, (uint32_t)f.dp, f.tgt);
-        tab[2 * threadIdx.x + 1] = make_uint4(f.add2, (uint32_t)f.dp2, f.mp, f.mm);
+        const ZFace f = zdir_face(zl, threadIdx.x, shift);
+        tab[2 * threadIdx.x] = make_uint4(f.m, f.add, f.mf, f.tgt);
+        tab[2 * threadIdx.x + 1] = make_uint4(f.add2, 0u, 0u, 0u);
     }
 }
 
@@ -172,49 +209,46 @@ __device__ __forceinline__ void zbuild_table_noflux(const ZLayout &zl, uint4 *ta
 // (zbuild_flag_key_table), fo = flags x 4096.
 struct ZEntry {
     uint32_t m, add, dp, fx, fy;      // axis mask, dilated addend, packed displacement, wrap fix-up
-    uint32_t tgt, add2, dp2, mp, mm;  // noflux: face test and the turned-around move (ZFlip)
+    uint32_t mf, tgt, add2;           // noflux: face test and the turned-around addend (ZFace)
 };
 
 // fo: the walker's table offset (mirror walks with reflection flags), else 0;
 // TAB 3: its key offset.
-template <bool WRAPFIX, int TAB = 0, bool NOFLUX = false>
-__device__ __forceinline__ void zdirection(uint64_t &s, const char *tab_bytes, const char *fix_bytes, ZEntry &e,
-                                           const uint8_t *keys = nullptr, uint32_t fo = 0u)
+template <int TAB>
+__device__ __forceinline__ uint32_t zdirection_key(uint64_t &s, const uint8_t *keys, uint32_t fo)
 {
-    static_assert(!NOFLUX || (TAB == 2 && !WRAPFIX), "noflux: byte-key table, no wrap fix-up");
-    static_assert(!(TAB == 1 && WRAPFIX), "the wide table has no wrap fix-up");
     s = xorshift64(s);
     const uint32_t lo = (uint32_t)s, hi = (uint32_t)(s >> 32);
-    uint32_t off;
-    if (TAB == 3) {
-        // the flags' key table: its offset is the key's accumulator
-        off = keys[zdot_key(lo, hi, fo)];
-    } else if (TAB == 2) {
-        off = keys[zdot_key(lo, hi, 0u)];
-    } else if (TAB == 1) {
-        // byte sum sb <= 2040 == state (mod 3)
-        const uint32_t sb = __builtin_amdgcn_sad_u8(hi, 0u, __builtin_amdgcn_sad_u8(lo, 0u, 0u));
-        off = (sb << 4) | ((lo << 15) & 0x8000u);
-    } else {
-        const uint32_t sb = __builtin_amdgcn_sad_u8(hi, 0u, __builtin_amdgcn_sad_u8(lo, 0u, 0u));
-        // q = sb / 3 by a 24-bit multiply; entry 2 * (sb - 3q) + (state & 1)
-        // at 16 bytes per entry
-        const uint32_t q = __umul24(sb, 2731u) >> 13;
-        off = (uint32_t)__mul24((int)q, -96) + ((sb << 5) | ((lo & 1u) << 4));
-    }
+    if (TAB == 3)   // the flags' key table: its offset is the key's accumulator
+        return keys[zdot_key(lo, hi, fo)];
+    if (TAB == 2)
+        return keys[zdot_key(lo, hi, 0u)];
+    // byte sum sb <= 2040 == state (mod 3)
+    const uint32_t sb = __builtin_amdgcn_sad_u8(hi, 0u, __builtin_amdgcn_sad_u8(lo, 0u, 0u));
+    if (TAB == 1)
+        return (sb << 4) | ((lo << 15) & 0x8000u);
+    // q = sb / 3 by a 24-bit multiply; entry 2 * (sb - 3q) + (state & 1)
+    // at 16 bytes per entry
+    const uint32_t q = __umul24(sb, 2731u) >> 13;
+    return (uint32_t)__mul24((int)q, -96) + ((sb << 5) | ((lo & 1u) << 4));
+}
+
+// The entry at the offset zdirection_key returned.
+template <bool WRAPFIX, int TAB, bool NOFLUX>
+__device__ __forceinline__ void zdirection_entry(uint32_t off, const char *tab_bytes, const char *fix_bytes, ZEntry &e,
+                                                 uint32_t fo)
+{
     if (TAB != 3)
         off += fo;
     const uint4 t = *reinterpret_cast<const uint4 *>(tab_bytes + off);
     e.m = t.x;
     e.add = t.y;
-    e.dp = t.z;
     if (NOFLUX) {
-        const uint4 u = *reinterpret_cast<const uint4 *>(tab_bytes + off + 16u);
+        e.mf = t.z;
         e.tgt = t.w;
-        e.add2 = u.x;
-        e.dp2 = u.y;
-        e.mp = u.z;
-        e.mm = u.w;
+        e.add2 = *reinterpret_cast<const uint32_t *>(tab_bytes + off + 16u);
+    } else {
+        e.dp = t.z;
     }
     if (WRAPFIX) {
         const uint2 f = *reinterpret_cast<const uint2 *>(fix_bytes + (off >> 1));
@@ -223,27 +257,26 @@ __device__ __forceinline__ void zdirection(uint64_t &s, const char *tab_bytes, c
     }
 }
 
-// Candidate address of the move of entry e from A (dilated add, periodic
-// wrap included; WRAPFIX: non-power-of-two period fix-up).
-template <bool WRAPFIX>
-__device__ __forceinline__ uint32_t zmove_entry(uint32_t A, const ZEntry &e)
+template <bool WRAPFIX, int TAB = 0, bool NOFLUX = false>
+__device__ __forceinline__ void zdirection(uint64_t &s, const char *tab_bytes, const char *fix_bytes, ZEntry &e,
+                                           const uint8_t *keys = nullptr, uint32_t fo = 0u)
 {
-    uint32_t c = (A & ~e.m) | (((A | ~e.m) + e.add) & e.m);
-    if (WRAPFIX)
-        c = (c & e.m) == e.fx ? ((c & ~e.m) | e.fy) : c;
-    return c;
+    static_assert(!NOFLUX || (TAB == 2 && !WRAPFIX), "noflux: byte-key table, no wrap fix-up");
+    static_assert(!(TAB == 1 && WRAPFIX), "the wide table has no wrap fix-up");
+    zdirection_entry<WRAPFIX, TAB, NOFLUX>(zdirection_key<TAB>(s, keys, fo), tab_bytes, fix_bytes, e, fo);
 }
 
-// Noflux candidate of entry e from A: the forward move, or the turned-around
-// one when the forward move crosses a face of the image; dp receives the
-// packed displacement of the move taken.
-__device__ __forceinline__ uint32_t zmove_noflux(uint32_t A, const ZEntry &e, int32_t &dp)
+// Candidate address of the move of entry e from A: the dilated add (its wrap
+// of power-of-two periods included), with WRAPFIX the wrap of other periods
+// and with NOFLUX the turn-around at a face, both tested on A beside the add.
+template <bool WRAPFIX, bool NOFLUX = false>
+__device__ __forceinline__ uint32_t zmove_entry(uint32_t A, const ZEntry &e)
 {
-    const uint32_t c = (A & ~e.m) | (((A | ~e.m) + e.add) & e.m);
-    const bool crossed = ((c & e.mp) | (A & e.mm)) == e.tgt;
-    const uint32_t cf = (A & ~e.m) | (((A | ~e.m) + e.add2) & e.m);
-    dp = (int32_t)(crossed ? e.dp2 : e.dp);
-    return crossed ? cf : c;
+    const uint32_t add = NOFLUX && (A & e.mf) == e.tgt ? e.add2 : e.add;
+    uint32_t f = (A | ~e.m) + add;
+    if (WRAPFIX)
+        f = (A & e.m) == e.fx ? e.fy : f;
+    return zsel(e.m, f, A);
 }
 
 // Candidate address of one move from A: advances the RNG state s, reads the
@@ -267,11 +300,12 @@ __device__ __forceinline__ uint32_t zpropose(uint64_t &s, uint32_t A, const char
     }
     const uint4 t = *reinterpret_cast<const uint4 *>(tab_bytes + off);
     const uint32_t m = t.x;
-    uint32_t c = (A & ~m) | (((A | ~m) + t.y) & m);
+    uint32_t f = (A | ~m) + t.y;
     if (WRAPFIX) {
-        const uint2 f = *reinterpret_cast<const uint2 *>(fix_bytes + (off >> 1));
-        c = (c & m) == f.x ? ((c & ~m) | f.y) : c;
+        const uint2 w = *reinterpret_cast<const uint2 *>(fix_bytes + (off >> 1));
+        f = (A & m) == w.x ? w.y : f;
     }
+    const uint32_t c = (A & ~m) | (f & m);
     dp = (int32_t)t.z;
     // keep the displacement in this one table read (the compiler would
     // otherwise re-read it inside the move branch)
@@ -352,17 +386,18 @@ __device__ __forceinline__ zv2u zchunk_load8(zrsrc_t rsrc, uint32_t cid)
 }
 #endif
 
-__device__ __forceinline__ zrsrc_t zchunk_rsrc(const uint32_t *words, const ZLayout &zl)
+// bits: address bits of the image's voxels
+__device__ __forceinline__ zrsrc_t zchunk_rsrc(const uint32_t *words, uint32_t bits)
 {
-    const int32_t chunks = (int32_t)(zl.bits > 7 ? (1u << (zl.bits - 7)) : 1u);   // 128 addresses each
+    const int32_t chunks = (int32_t)(bits > 7 ? (1u << (bits - 7)) : 1u);   // 128 addresses each
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t *>(words), (short)16, chunks, kZChunkRsrcWord3);
 }
 
 // The same over the image's 8-byte chunks (4 x 4 x 4 voxels, 64 addresses;
 // stride 8, num_records = that chunk count).
-__device__ __forceinline__ zrsrc_t zchunk_rsrc8(const uint32_t *words, const ZLayout &zl)
+__device__ __forceinline__ zrsrc_t zchunk_rsrc8(const uint32_t *words, uint32_t bits)
 {
-    const int32_t chunks = (int32_t)(zl.bits > 6 ? (1u << (zl.bits - 6)) : 1u);
+    const int32_t chunks = (int32_t)(bits > 6 ? (1u << (bits - 6)) : 1u);
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t *>(words), (short)8, chunks, kZChunkRsrcWord3);
 }
 
@@ -391,26 +426,18 @@ __device__ __forceinline__ void zchunk_fill_buf(const zrsrc_t &rsrc, uint32_t c,
     QB = cid;
 }
 
+// All ones when address c's voxel is solid (its bit in the chunk QV), else 0.
 template <int CW>
 __device__ __forceinline__ uint32_t zchunk_wall(uint32_t c, const uint4 &QV)
 {
     uint64_t half = ((uint64_t)QV.y << 32) | QV.x;
     if (CW == 128) {
-        // the half that bit 6 of c selects, by two bitfield inserts under the
-        // sign-extended bit (3 VALU; a compare and two selects take 4)
-        // (as inline VALU: the compiler turns the mask form back into selects)
+        // the half that bit 6 of c selects, under the sign-extended bit
         const uint32_t sel = (uint32_t)__builtin_amdgcn_sbfe((int)c, 6u, 1u);
-        uint32_t lo, hi;
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(lo) : "v"(sel), "v"(QV.z), "v"(QV.x));
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(hi) : "v"(sel), "v"(QV.w), "v"(QV.y));
-        half = ((uint64_t)hi << 32) | lo;
+        half = ((uint64_t)zsel(sel, QV.w, QV.y) << 32) | zsel(sel, QV.z, QV.x);
     }
-    // descending bit order: address c's bit is bit 63 - (c & 63); the empty
-    // asm keeps the sign test on the high word (the compiler would widen it
-    // to a 64-bit compare)
-    uint32_t top = (uint32_t)((half << (c & 63u)) >> 32);
-    asm("" : "+v"(top));
-    return top >> 31;
+    // descending bit order: address c's bit is bit 63 - (c & 63)
+    return (uint32_t)((int32_t)(uint32_t)((half << (c & 63u)) >> 32) >> 31);
 }
 
 // Label-volume address of address c: the first-octant address when
@@ -485,11 +512,15 @@ __device__ __forceinline__ uint32_t zcompact(uint32_t v, uint32_t m)
 // last flush (per axis, the coordinate change taken modulo the period into
 // (-period / 2, period / 2), negated along reflected axes), one VALU per
 // move fewer.
+// SUB: voxel division by 2^a.shift (one walker per lane): a.zl addresses
+// sub-voxels, interleaved like the image's voxels above the low 3 a.shift
+// bits, so the voxel address is a shift of the sub-voxel one (1 VALU per
+// step more) and the image is the undivided one.
 // HITS false (CPMG, a.hits null): no wall-hit count, as the reference's
 // CPMG kernels (NMR_cpmg_cuda.cpp:380-386: a hit only multiplies the
 // energy), one VALU per step fewer.
 template <int EMODE, int K, bool WRAPFIX, int CACHE, int TAB = 0, bool NOFLUX = false, bool MFLAGS = false,
-          int NS = 1, bool JAC = false, bool ADISP = false, bool HITS = true>
+          int NS = 1, bool JAC = false, bool ADISP = false, bool HITS = true, bool SUB = false>
 __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, double *part, uint64_t part_stride,
                                            double (*lds)[kEchoCols], const uint4 *tab, const uint2 *fix,
                                            const double *ldelta = nullptr, const uint8_t *keys = nullptr,
@@ -502,11 +533,15 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     static_assert(NS == 1 || (NS == 8 && EMODE == 2 && K == 1 && CACHE >= 64), "label sets: 8 sets, K == 1");
     static_assert(!ADISP || (MFLAGS && !NOFLUX && CACHE >= 64), "address displacements: pipelined mirror walk");
     static_assert(HITS || (EMODE == 1 && CACHE >= 64), "uncounted hits: pipelined CPMG walk");
+    static_assert(!SUB || (CACHE == 128 && K == 1), "voxel division: pipelined walk of one walker per lane");
+    const uint32_t sub = SUB ? (uint32_t)a.shift : 0u, sub3 = 3u * sub;
+    auto voxel = [&](uint32_t c) { return SUB ? c >> sub3 : c; };
     // label-set walks count no per-label hits (a.label_hits is null)
     constexpr bool LH_LDS = EMODE == 2 && K == 1 && NS == 1;
     constexpr int NL = (EMODE == 2 && !LH_LDS && NS == 1) ? kMaxLabels : 1;
     const char *words = reinterpret_cast<const char *>(a.zwords);
-    const zrsrc_t zrsrc = CACHE == 64 ? zchunk_rsrc8(a.zwords, a.zl) : zchunk_rsrc(a.zwords, a.zl);
+    const zrsrc_t zrsrc =
+        CACHE == 64 ? zchunk_rsrc8(a.zwords, a.zl.bits) : zchunk_rsrc(a.zwords, a.zl.bits - sub3);
     // the tile's walkers: blockDim x K from tile x blockDim x K, or with
     // balanced tiles a.tile_walkers (at most blockDim, K == 1) from tile x
     // a.tile_walkers
@@ -543,7 +578,8 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
         Y[k] = act[k] ? a.y[j] : 0;
         Z[k] = act[k] ? a.z[j] : 0;
         if (NOFLUX && act[k] &&
-            !((unsigned)X[k] < (unsigned)a.W && (unsigned)Y[k] < (unsigned)a.H && (unsigned)Z[k] < (unsigned)a.D)) {
+            !((unsigned)(X[k] >> sub) < (unsigned)a.W && (unsigned)(Y[k] >> sub) < (unsigned)a.H &&
+              (unsigned)(Z[k] >> sub) < (unsigned)a.D)) {
             // a noflux walker must start inside the image (as the folded walk)
             act[k] = false;
             atomicOr(a.error_flag, 1u);
@@ -596,7 +632,12 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
         static_for<K>([&](auto kc) {
             constexpr int k = decltype(kc)::value;
             int32_t dx, dy, dz;
-            if constexpr (ADISP) {
+            if constexpr (NOFLUX) {
+                // the walker never left the image: its coordinates are its address
+                dx = (int32_t)zcompact(A[k], a.zl.m[0]) - X[k];
+                dy = (int32_t)zcompact(A[k], a.zl.m[1]) - Y[k];
+                dz = (int32_t)zcompact(A[k], a.zl.m[2]) - Z[k];
+            } else if constexpr (ADISP) {
                 const uint32_t flags = FO[k] / (TAB == 3 ? kZKeyEntries : kZFlagStride);
                 int32_t d[3];
 #pragma unroll
@@ -628,6 +669,8 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     // between the chunk load of a step and its use, so the RNG, the table
     // read and the load overlap; the state is rewound by one step at the end.
     constexpr bool PIPE = CACHE >= 64;
+    // moves added to a packed displacement (not where the address tells them)
+    constexpr bool DISP = !ADISP && !NOFLUX;
     ZEntry T[K];
     if (PIPE)
         static_for<K>([&](auto kc) {
@@ -670,11 +713,10 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     auto step = [&]() {
         static_for<K>([&](auto kc) {
             constexpr int k = decltype(kc)::value;
-            if (NOFLUX) {
-                C[k] = zmove_noflux(A[k], T[k], DP[k]);
-            } else if (PIPE) {
-                C[k] = zmove_entry<WRAPFIX>(A[k], T[k]);
-                DP[k] = (int32_t)T[k].dp;
+            if (PIPE) {
+                C[k] = zmove_entry<WRAPFIX, NOFLUX>(A[k], T[k]);
+                if (!NOFLUX)
+                    DP[k] = (int32_t)T[k].dp;
             } else {
                 C[k] = zpropose<WRAPFIX, WIDE>(S[k], A[k], tab_bytes, fix_bytes, DP[k]);
             }
@@ -695,7 +737,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
             static_for<K>([&](auto kc) {
                 constexpr int k = decltype(kc)::value;
                 if (CACHE == 128)
-                    zchunk_fill_buf(zrsrc, C[k], QB[k], QV[k]);
+                    zchunk_fill_buf(zrsrc, voxel(C[k]), QB[k], QV[k]);
                 else
                     zchunk_fill_buf8(zrsrc, C[k], QB[k], QV[k]);
             });
@@ -710,7 +752,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
             settle_labels();
             static_for<K>([&](auto kc) {
                 constexpr int k = decltype(kc)::value;
-                wallv[k] = zchunk_wall<CACHE == 64 ? 64 : 128>(C[k], QV[k]);
+                wallv[k] = zchunk_wall<CACHE == 64 ? 64 : 128>(voxel(C[k]), QV[k]);
             });
         } else {
             static_for<K>([&](auto kc) {
@@ -724,42 +766,42 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
         static_for<K>([&](auto kc) {
             constexpr int k = decltype(kc)::value;
             const uint32_t wall = wallv[k];
-            if (CACHE >= 64 && EMODE == 1) {
-                // two short divergent paths (4 VALU in all) instead of the
-                // selects and unconditional multiply the compiler would make
+            if (CACHE >= 64 && DISP && EMODE == 1) {
+                // a packed displacement to keep as well: two short divergent
+                // paths (3-5% faster than masks from 5 waves per SIMD on)
                 if (__builtin_expect(wall != 0u, 0)) {
                     if (HITS)
                         Hc[k] += 1u;
                     E[k] *= DL[k];
                 } else {
                     A[k] = C[k];
-                    if (!ADISP)
-                        P[k] += DP[k];
-                    else   // a move of one copy: kept a branch, not turned into selects
-                        asm volatile("" : "+v"(A[k]));
+                    P[k] += DP[k];
                 }
                 return;
             }
-            if (CACHE >= 64 && EMODE == 2) {
-                if (__builtin_expect(wall != 0u, 0)) {
-                    Hc[k] += 1u;
-                    PW[k] = zlabel_at(a, C[k]);
+            if (CACHE >= 64) {
+                // wall is a mask here: no branch but the label's load
+                A[k] = zsel(wall, A[k], C[k]);
+                if (DISP)
+                    P[k] += (int32_t)((uint32_t)DP[k] & ~wall);
+                if (HITS)
+                    Hc[k] -= wall;
+                if (EMODE == 1)
+                    E[k] = zsel_f64(wall, E[k] * DL[k], E[k]);
+                if (EMODE == 2 && __builtin_expect(wall != 0u, 0)) {
+                    PW[k] = zlabel_at(a, voxel(C[k]));
                     PEND[k] = true;
-                } else {
-                    A[k] = C[k];
-                    if (!ADISP)
-                        P[k] += DP[k];
                 }
                 return;
             }
             A[k] = wall ? A[k] : C[k];
-            if (!ADISP)
+            if (DISP)
                 P[k] += wall ? 0 : DP[k];
             Hc[k] += wall;
             if (EMODE == 1 && wall)
                 E[k] *= DL[k];
             if (EMODE == 2 && wall) {
-                const uint32_t lab = zlabel_at(a, C[k]);
+                const uint32_t lab = zlabel_at(a, voxel(C[k]));
                 E[k] *= ldelta[lab];
                 if (LH_LDS) {
                     __hip_atomic_fetch_add(my_lh + lab, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -778,7 +820,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     auto walk_echo = [&]() {
         uint32_t left = spe;
         while (left) {
-            const uint32_t ns = left < kZFlush - since ? left : kZFlush - since;
+            const uint32_t ns = NOFLUX || left < kZFlush - since ? left : kZFlush - since;
             // two steps per trip: the pipelined direction entry then lives in
             // alternating registers instead of being copied every step
             uint32_t i = 0;
@@ -790,7 +832,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
                 step();
             since += ns;
             left -= ns;
-            if (since == kZFlush) {
+            if (!NOFLUX && since == kZFlush) {
                 flush();
                 since = 0;
             }
@@ -872,29 +914,94 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     });
 }
 
-// Speculative CPMG tile for latency-bound runs (few waves per SIMD, where a
-// step waits for its chunk load with nothing else to issue): one walker per
-// lane, no chunk cache, directions drawn two steps ahead.  At the start of
-// step t both possible candidates of step t + 1 are formed, from the current
-// position (if step t hits a wall) and from step t's candidate (if it
-// moves), and both of their 16-byte chunks are loaded; then the direction of
-// step t + 2 is drawn, and only then does step t wait for its own chunk,
-// loaded at the start of step t - 1 (the empty asm holds that wait after the
-// draw).  Two chunk loads per walker-step (more VALU and L2 requests than
-// the chunk-cache walk), so it pays only when the walk is latency-bound.
-// Same walk, bit for bit, as zwalk_tile (EMODE 1).
-template <bool WRAPFIX, bool NOFLUX, bool MFLAGS>
+// Echo sums of the speculative tile.  With one wave per SIMD an instruction
+// costs 5 cycles or more whatever it does, so the lanes' values are not summed
+// across the wave echo by echo (about 10 instructions each, run_echoes): a lane
+// writes its value into a row of LDS (one row of 64 per echo, padded to
+// kZRowStride so that the reads below spread over the banks), and every 8
+// echoes lane 8 e + q adds the 8 values q, q + 8, ... of row e, then the 8
+// partial sums of a row meet in lane 8 e: 3.3 instructions per echo and the
+// write.  Fixed order, so deterministic.
+constexpr uint32_t kZRowEchoes = 8u, kZRowStride = 72u;
+
+struct ZEchoRows {
+    double *rows;               // this wave's kZRowEchoes x kZRowStride
+    double (*lds)[kEchoCols];   // wave totals of kEchoChunk echoes (blocks of several waves)
+    double *out;
+    uint64_t row_stride;
+    uint32_t last;              // last echo
+
+    // Stage v for `echo`; all threads of the block call it, echoes in order.
+    __device__ __forceinline__ void put(uint32_t echo, double v) const
+    {
+        const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, nw = blockDim.x / kWave;
+        rows[(echo % kZRowEchoes) * kZRowStride + lane] = v;
+        if (echo % kZRowEchoes != kZRowEchoes - 1u && echo != last)
+            return;
+        // the rows were written by this wave: its LDS accesses stay in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const double *r = rows + (lane >> 3) * kZRowStride + (lane & 7u);
+        double s = r[0];
+#pragma unroll
+        for (uint32_t i = 1; i < 8u; ++i)
+            s += r[8u * i];
+        s += dpp_f64<0xB1>(s);    // lane ^ 1
+        s += dpp_f64<0x4E>(s);    // lane ^ 2
+        s += dpp_f64<0x141>(s);   // half-row mirror
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t first = echo - echo % kZRowEchoes, e = first + (lane >> 3);
+        const bool mine = (lane & 7u) == 0u && e <= echo;   // rows past the last echo hold no values
+        if (nw == 1u) {
+            if (mine)
+                out[(uint64_t)e * row_stride] = s;
+            return;
+        }
+        static_assert(kEchoChunk % kZRowEchoes == 0, "whole groups of rows per chunk");
+        if (mine)
+            lds[e % kEchoChunk][wave] = s;
+        const uint32_t slot = echo % kEchoChunk;
+        if (slot == kEchoChunk - 1 || echo == last) {
+            __syncthreads();
+            if (threadIdx.x <= slot) {
+                double sum = 0.0;
+                for (uint32_t q = 0; q < nw; ++q)
+                    sum += lds[threadIdx.x][q];
+                out[(uint64_t)(echo - slot + threadIdx.x) * row_stride] = sum;
+            }
+            __syncthreads();
+        }
+    }
+};
+
+// Speculative tile for latency-bound runs (few waves per SIMD, where a step
+// of the chunk-cache walk waits for its chunk load with nothing else to
+// issue): one walker per lane, no chunk cache.  At the start of step t both
+// possible candidates of step t + 1 are formed, from the current position
+// (step t hits a wall) and from step t's candidate (it moves), and the 8-byte
+// words that hold their bits are loaded; then step t is resolved from the
+// words loaded at the start of step t - 1.  So a load has a step and a half
+// to arrive.  The directions run ahead too: at step t the entry of step t + 2
+// is read from the table, through the key byte read a step earlier, and the
+// key of step t + 3 is drawn, so neither table read is waited for.  A step is
+// free of branches: a hit multiplies the energy by delta, a move by 1.0.
+// Same walk, bit for bit, as zwalk_tile (EMODE 0 and 1; SUB as there).
+template <int EMODE, bool WRAPFIX, bool NOFLUX, bool MFLAGS, bool SUB>
 __device__ __forceinline__ void zwalk_tile_spec(const WalkArgs &a, uint64_t tile, double *part, uint64_t part_stride,
-                                                double (*lds)[kEchoCols], const uint4 *tab, const uint2 *fix,
-                                                const uint8_t *keys)
+                                                double (*lds)[kEchoCols], double *rows, const uint4 *tab,
+                                                const uint2 *fix, const uint8_t *keys)
 {
-    const zrsrc_t zrsrc = zchunk_rsrc(a.zwords, a.zl);
+    const uint32_t sub = SUB ? (uint32_t)a.shift : 0u, sub3 = 3u * sub;
+    const zrsrc_t zrsrc = zchunk_rsrc8(a.zwords, a.zl.bits - sub3);
     const uint64_t id = tile * blockDim.x + threadIdx.x;
     const uint32_t echoes = a.echoes, spe = a.steps_per_echo;
     bool act = id < a.n;
     const uint64_t j = act ? id : 0;
     int32_t X = act ? a.x[j] : 0, Y = act ? a.y[j] : 0, Z = act ? a.z[j] : 0;
-    if (NOFLUX && act && !((unsigned)X < (unsigned)a.W && (unsigned)Y < (unsigned)a.H && (unsigned)Z < (unsigned)a.D)) {
+    if (NOFLUX && act &&
+        !((unsigned)(X >> sub) < (unsigned)a.W && (unsigned)(Y >> sub) < (unsigned)a.H &&
+          (unsigned)(Z >> sub) < (unsigned)a.D)) {
         act = false;   // a noflux walker must start inside the image
         atomicOr(a.error_flag, 1u);
         X = Y = Z = 0;
@@ -916,91 +1023,163 @@ __device__ __forceinline__ void zwalk_tile_spec(const WalkArgs &a, uint64_t tile
     int32_t P = 0;
     const char *tab_bytes = reinterpret_cast<const char *>(tab);
     const char *fix_bytes = reinterpret_cast<const char *>(fix);
-    auto move = [&](uint32_t from, const ZEntry &t, int32_t &dp) -> uint32_t {
-        if (NOFLUX)
-            return zmove_noflux(from, t, dp);
-        dp = (int32_t)t.dp;
-        return zmove_entry<WRAPFIX>(from, t);
+    auto word = [&](uint32_t c) -> uint64_t {   // the 8-byte word of address c's voxel
+        const zv2u v = zchunk_load8(zrsrc, c >> (sub3 + 6u));
+        return ((uint64_t)v.y << 32) | v.x;
     };
-    auto chunk = [&](uint32_t c) -> uint4 {
-        const zv4u v = zchunk_load(zrsrc, c >> 7);
-        return make_uint4(v.x, v.y, v.z, v.w);
-    };
-    // the first step's candidate C and its chunk (in both slots), and the
-    // second step's direction T
-    ZEntry T;
-    zdirection<WRAPFIX, 2, NOFLUX>(S, tab_bytes, fix_bytes, T, keys, FO);
-    int32_t DP;
-    uint32_t C = move(A, T, DP);
-    uint4 QS = chunk(C), QM = chunk(C);
-    bool stay = true;   // which of QS / QM holds the chunk of C
-    zdirection<WRAPFIX, 2, NOFLUX>(S, tab_bytes, fix_bytes, T, keys, FO);
-    auto step = [&]() {
-        int32_t dps, dpm;
-        const uint32_t cs = move(A, T, dps);   // next candidate if this step hits
-        const uint32_t cm = move(C, T, dpm);   // next candidate if this step moves
-        const uint4 qs = chunk(cs);
-        const uint4 qm = chunk(cm);
-        ZEntry Tn;
-        zdirection<WRAPFIX, 2, NOFLUX>(S, tab_bytes, fix_bytes, Tn, keys, FO);
-        // this step's chunks were loaded a step ago: wait for them here,
-        // after the loads above and the draw, not before
-        asm volatile("" : "+v"(QS.x), "+v"(QS.y), "+v"(QS.z), "+v"(QS.w), "+v"(QM.x), "+v"(QM.y), "+v"(QM.z),
-                     "+v"(QM.w)::"memory");
-        const uint4 q = stay ? QS : QM;
-        const bool wall = zchunk_wall<128>(C, q) != 0u;
-        if (__builtin_expect(wall, 0)) {
-            Hc += 1u;
-            E *= DL;
-        } else {
-            A = C;
-            P += DP;
+    // Two register sets, so that what a step loads for the next one is never
+    // copied: step<p> uses T[p], QS[p] and QM[p] and fills those of p ^ 1.
+    // T[p]: the next step's direction; QS[p] / QM[p]: the words of this
+    // step's candidate C, loaded in case the step before hit or moved
+    // (`stay`, a mask: it hit); T[p ^ 1].dp until it is refilled: C's displacement.
+    ZEntry T[2];
+    uint64_t QS[2], QM[2];
+    zdirection<WRAPFIX, 2, NOFLUX>(S, tab_bytes, fix_bytes, T[1], keys, FO);
+    uint32_t C = zmove_entry<WRAPFIX, NOFLUX>(A, T[1]);
+    QS[0] = QM[0] = word(C);
+    uint32_t stay = 0xFFFFFFFFu;
+    zdirection<WRAPFIX, 2, NOFLUX>(S, tab_bytes, fix_bytes, T[0], keys, FO);
+    uint32_t off = zdirection_key<2>(S, keys, FO);
+    // One wave issues an instruction every 4 cycles, but a dependent one only
+    // after about 8, so the serial xorshift is laid beside the two moves and
+    // the wall test, a few independent instructions at a time; the barriers
+    // keep the compiler from putting the chains one after another (128^3, 10k
+    // walkers, 12 steps per echo: 117 -> 106 ns per step).
+#define ZSPEC_KEEP() __builtin_amdgcn_sched_barrier(0)
+    auto step = [&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        const ZEntry &t = T[p];
+        uint64_t s = S, r;
+        uint32_t adds = t.add, addm = t.add;
+        r = s << 13;
+        const int32_t pd = NOFLUX ? 0 : P + (int32_t)T[p ^ 1].dp;
+        if (NOFLUX) {
+            adds = (A & t.mf) == t.tgt ? t.add2 : t.add;
+            addm = (C & t.mf) == t.tgt ? t.add2 : t.add;
         }
-        C = wall ? cs : cm;
-        DP = wall ? dps : dpm;
-        QS = qs;
-        QM = qm;
+        uint32_t fs = A | ~t.m, fm = C | ~t.m;
+        ZSPEC_KEEP();
+        s ^= r;
+        fs += adds;
+        fm += addm;
+        ZSPEC_KEEP();
+        r = s >> 7;
+        if (WRAPFIX) {
+            fs = (A & t.m) == t.fx ? t.fy : fs;
+            fm = (C & t.m) == t.fx ? t.fy : fm;
+        }
+        const uint32_t cs = zsel(t.m, fs, A);   // next candidate if this step hits
+        const uint32_t cm = zsel(t.m, fm, C);   // next candidate if this step moves
+        ZSPEC_KEEP();
+        s ^= r;
+        const uint32_t is = cs >> (sub3 + 6u), im = cm >> (sub3 + 6u);
+        ZSPEC_KEEP();
+        const zv2u ws = zchunk_load8(zrsrc, is);
+        const zv2u wm = zchunk_load8(zrsrc, im);
+        r = s << 17;
+        zdirection_entry<WRAPFIX, 2, NOFLUX>(off, tab_bytes, fix_bytes, T[p ^ 1], FO);
+        ZSPEC_KEEP();
+        s ^= r;
+        // this step's words were loaded a step ago
+        const uint64_t q = zsel64(stay, QS[p], QM[p]);
+        const uint32_t v = SUB ? C >> sub3 : C;
+        ZSPEC_KEEP();
+        const uint32_t kh = __builtin_amdgcn_udot4((uint32_t)(s >> 32), kZKeyWeightsHi, 0u, false);
+        // the bit of address v is bit 63 - (v & 63) of its word
+        const uint32_t top = (uint32_t)((q << (v & 63u)) >> 32);
+        const double eh = EMODE == 1 ? E * DL : E;
+        ZSPEC_KEEP();
+        const uint32_t key = __builtin_amdgcn_udot4((uint32_t)s, kZKeyWeightsLo, kh, false);
+        const uint32_t wall = (uint32_t)((int32_t)top >> 31);
+        ZSPEC_KEEP();
+        A = zsel(wall, A, C);
+        C = zsel(wall, cs, cm);
+        off = keys[key];
+        ZSPEC_KEEP();
+        Hc -= wall;
+        if (EMODE == 1)
+            E = zsel_f64(wall, eh, E);
+        if (!NOFLUX)
+            P = (int32_t)zsel(wall, (uint32_t)P, (uint32_t)pd);
+        S = s;
+        QS[p ^ 1] = ((uint64_t)ws.y << 32) | ws.x;
+        QM[p ^ 1] = ((uint64_t)wm.y << 32) | wm.x;
         stay = wall;
-        T = Tn;
     };
+#undef ZSPEC_KEEP
     uint32_t since = 0;
     auto flush = [&]() {
+        if (NOFLUX) {
+            // the walker never left the image: its coordinates are its address
+            X = (int32_t)zcompact(A, a.zl.m[0]);
+            Y = (int32_t)zcompact(A, a.zl.m[1]);
+            Z = (int32_t)zcompact(A, a.zl.m[2]);
+            return;
+        }
         int32_t dx, dy, dz;
         zunpack(P, dx, dy, dz);
         X += dx;
         Y += dy;
         Z += dz;
         P = 0;
+        since = 0;
     };
-    auto walk_echo = [&]() {
+    // Steps of one echo, entered with register set p: pairs of steps, then
+    // one more when their number is odd (the next echo enters with p ^ 1; it
+    // stands after every loop, so no wait for its loads lies inside one).
+    constexpr uint32_t kRun = kZFlush - 1u;   // even
+    auto walk_steps = [&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        auto pairs = [&](uint32_t ns) {
+            if (!NOFLUX) {
+                if (since + ns > kZFlush)
+                    flush();
+                since += ns;
+            }
+            for (uint32_t i = ns >> 1; i; --i) {
+                step(std::integral_constant<int, p>{});
+                step(std::integral_constant<int, p ^ 1>{});
+            }
+        };
         uint32_t left = spe;
-        while (left) {
-            const uint32_t ns = left < kZFlush - since ? left : kZFlush - since;
-            uint32_t i = 0;
-            for (; i + 2 <= ns; i += 2) {
-                step();
-                step();
-            }
-            if (i < ns)
-                step();
-            since += ns;
-            left -= ns;
-            if (since == kZFlush) {
-                flush();
-                since = 0;
-            }
-        }
+        if (!NOFLUX)
+            for (; left > kRun; left -= kRun)
+                pairs(kRun);
+        pairs(left);
+        if (left & 1u)
+            step(std::integral_constant<int, p>{});
     };
-    run_echoes<true>(echoes, lds, part, part_stride, walk_echo, [&]() { return E; });
+    const ZEchoRows er{rows + (threadIdx.x / kWave) * (kZRowEchoes * kZRowStride), lds, part, part_stride, echoes};
+    if (part)
+        er.put(0, E);
+    if (spe & 1u) {
+        // an odd number of steps: the echoes alternate between the sets
+        for (uint32_t echo = 1; echo <= echoes; echo += 2) {
+            walk_steps(std::integral_constant<int, 0>{});
+            if (part)
+                er.put(echo, E);
+            if (echo == echoes)
+                break;
+            walk_steps(std::integral_constant<int, 1>{});
+            if (part)
+                er.put(echo + 1, E);
+        }
+    } else {
+        for (uint32_t echo = 1; echo <= echoes; ++echo) {
+            walk_steps(std::integral_constant<int, 0>{});
+            if (part)
+                er.put(echo, E);
+        }
+    }
     flush();
-    // the directions were drawn two steps ahead
-    S = xorshift64_inverse(xorshift64_inverse(S));
+    // the directions were drawn three steps ahead
+    S = xorshift64_inverse(xorshift64_inverse(xorshift64_inverse(S)));
     if (act) {
         a.x[id] = X;
         a.y[id] = Y;
         a.z[id] = Z;
         a.seed[id] = S;
-        if (a.energy)
+        if (EMODE == 1 && a.energy)
             a.energy[id] = E;
         if (a.hits)
             a.hits[id] = Hc;

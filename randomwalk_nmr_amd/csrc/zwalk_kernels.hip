@@ -23,7 +23,7 @@ hipError_t launch_z_mode(const WalkArgs &a, const LaunchShape &ls, uint32_t bloc
 // interleave, so each wave keeps K chunk reloads in flight, and their
 // measurement terms are added in the lane before the cross-lane sums.
 // NOFLUX: noflux walk on the periodic unfolded image (face test and
-// turn-around, zmove_noflux); walkers must start inside the image.  MAXSETS:
+// turn-around, zmove_entry); walkers must start inside the image.  MAXSETS:
 // the most energy sets the instance handles (1, 2 or kMaxSets; registers).
 // Two walkers per lane fit 168 VGPRs (3 waves per SIMD) for rotation k rows,
 // up to two sets and the periodic / mirror walk; the other instances take
@@ -35,7 +35,7 @@ __global__ __launch_bounds__(kPfgseThreads, (K > 1 && ROT && MAXSETS <= 2 && !NO
     __shared__ double lds[kMaxSets * kPfgseKChunk][kPfgseWaves];
     __shared__ uint4 tab[NOFLUX ? 12 : 6];
     __shared__ uint2 fix[6];
-    __shared__ uint8_t keys[kZKeyEntries];
+    __shared__ __align__(16) uint8_t keys[kZKeyEntries];
     if (NOFLUX)
         zbuild_table_noflux(a.zl, tab);
     else
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kPfgseThreads, (K > 1 && ROT && MAXSETS <= 2 && !NO
     uint4 QV[K];
     double own_delta[K], e[K][MAXSETS];
     ZEntry T[K];
-    const zrsrc_t zrsrc = zchunk_rsrc(a.zwords, a.zl);
+    const zrsrc_t zrsrc = zchunk_rsrc(a.zwords, a.zl.bits);
     const char *tab_bytes = reinterpret_cast<const char *>(tab);
     const char *fix_bytes = reinterpret_cast<const char *>(fix);
     static_for<K>([&](auto kc) {
@@ -92,6 +92,13 @@ __global__ __launch_bounds__(kPfgseThreads, (K > 1 && ROT && MAXSETS <= 2 && !NO
     auto flush = [&]() {
         static_for<K>([&](auto kc) {
             constexpr int k = decltype(kc)::value;
+            if (NOFLUX) {
+                // the walker never left the image: its coordinates are its address
+                X[k] = (int32_t)zcompact(A[k], a.zl.m[0]);
+                Y[k] = (int32_t)zcompact(A[k], a.zl.m[1]);
+                Z[k] = (int32_t)zcompact(A[k], a.zl.m[2]);
+                return;
+            }
             int32_t dx, dy, dz;
             zunpack(P[k], dx, dy, dz);
             X[k] += dx;
@@ -109,12 +116,8 @@ __global__ __launch_bounds__(kPfgseThreads, (K > 1 && ROT && MAXSETS <= 2 && !NO
             int32_t dp[K];
             static_for<K>([&](auto kc) {
                 constexpr int k = decltype(kc)::value;
-                if (NOFLUX) {
-                    c[k] = zmove_noflux(A[k], T[k], dp[k]);
-                } else {
-                    c[k] = zmove_entry<WRAPFIX>(A[k], T[k]);
-                    dp[k] = (int32_t)T[k].dp;
-                }
+                c[k] = zmove_entry<WRAPFIX, NOFLUX>(A[k], T[k]);
+                dp[k] = NOFLUX ? 0 : (int32_t)T[k].dp;
                 zchunk_fill_buf(zrsrc, c[k], QB[k], QV[k]);
             });
             static_for<K>([&](auto kc) {
@@ -126,17 +129,15 @@ __global__ __launch_bounds__(kPfgseThreads, (K > 1 && ROT && MAXSETS <= 2 && !NO
             __builtin_amdgcn_sched_barrier(0);
             static_for<K>([&](auto kc) {
                 constexpr int k = decltype(kc)::value;
-                // two short divergent paths instead of selects
-                if (__builtin_expect(zchunk_wall<128>(c[k], QV[k]) != 0u, 0)) {
-                    H[k] += 1u;
-                } else {
-                    A[k] = c[k];
-                    P[k] += dp[k];
-                }
+                const uint32_t wall = zchunk_wall<128>(c[k], QV[k]);
+                H[k] -= wall;
+                A[k] = zsel(wall, A[k], c[k]);
+                if (!NOFLUX)
+                    P[k] += (int32_t)((uint32_t)dp[k] & ~wall);
             });
         };
         while (left) {
-            const uint32_t ns = left < kZFlush - since ? left : kZFlush - since;
+            const uint32_t ns = NOFLUX || left < kZFlush - since ? left : kZFlush - since;
             // two steps per trip (the pipelined entry alternates registers)
             uint32_t st = 0;
             for (; st + 2 <= ns; st += 2) {
@@ -147,7 +148,7 @@ __global__ __launch_bounds__(kPfgseThreads, (K > 1 && ROT && MAXSETS <= 2 && !NO
                 step();
             since += ns;
             left -= ns;
-            if (since == kZFlush)
+            if (!NOFLUX && since == kZFlush)
                 flush();
         }
         flush();
@@ -325,10 +326,9 @@ hipError_t launch_zwalk(const WalkArgs &a, int emode, const LaunchShape &ls, hip
 {
     if (a.n == 0)
         return hipSuccess;
-    if (a.shift != 0 || a.zwords == nullptr || ls.threads > max_threads_for_k((int)ls.k) || ls.threads % 64 != 0 ||
-        ls.threads == 0)
+    if (a.zwords == nullptr || ls.threads > max_threads_for_k((int)ls.k) || ls.threads % 64 != 0 || ls.threads == 0)
         return hipErrorInvalidValue;
-    const uint64_t per_block = (uint64_t)ls.threads * ls.k;
+    const uint64_t per_block = a.shift ? (uint64_t)ls.threads : (uint64_t)ls.threads * ls.k;
     uint64_t tiles = (a.n + per_block - 1) / per_block;
     if (a.tile_walkers) {
         // balanced tiles: only for the address-displacement mirror walk, one

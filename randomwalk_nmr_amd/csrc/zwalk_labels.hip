@@ -16,7 +16,7 @@ __global__ __launch_bounds__(1024) void zwalk_sets_kernel(const WalkArgs a)
     extern __shared__ double lds8[];   // kEchoChunk x 8 sets x waves of the block
     __shared__ uint4 tab[MFLAGS ? 8 * kZFlagStride / 16 : (NOFLUX ? 12 : 6)];
     __shared__ uint2 fix[MFLAGS ? 8 * kZFlagStride / 16 : 6];
-    __shared__ uint8_t keys[kZKeyEntries];
+    __shared__ __align__(16) uint8_t keys[kZKeyEntries];
     __shared__ double ldelta[8 * kMaxLabels];
     const uint64_t tile = tile_of_block(a);
     if (a.tile_map && tile >= a.n_tiles)
@@ -49,7 +49,7 @@ __global__ __launch_bounds__(1024) void zwalk_jac_kernel(const WalkArgs a)
     __shared__ double lds[kEchoChunk][kEchoCols];
     __shared__ uint4 tab[MFLAGS ? 8 * kZFlagStride / 16 : (NOFLUX ? 12 : 6)];
     __shared__ uint2 fix[MFLAGS ? 8 * kZFlagStride / 16 : 6];
-    __shared__ uint8_t keys[kZKeyEntries];
+    __shared__ __align__(16) uint8_t keys[kZKeyEntries];
     __shared__ double ldelta[kMaxLabels];
     const uint64_t tile = tile_of_block(a);
     if (a.tile_map && tile >= a.n_tiles)

@@ -13,11 +13,12 @@
 
 namespace rwnmr {
 
-// The speculative CPMG walk (zwalk_spec.hip), one walker per lane.
-hipError_t launch_z_spec(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st);
+// The speculative CPMG (emode 1) and map (0) walks (zwalk_spec.hip), one
+// walker per lane.
+hipError_t launch_z_spec(const WalkArgs &a, int emode, const LaunchShape &ls, uint32_t blocks, hipStream_t st);
 
 template <int EMODE, int K, bool WRAPFIX, int CACHE, int TAB, bool NOFLUX = false, bool MFLAGS = false,
-          bool ADISP = false, bool HITS = true>
+          bool ADISP = false, bool HITS = true, bool SUB = false>
 __global__ __launch_bounds__(max_threads_for_k(K)) void zwalk_kernel(const WalkArgs a)
 {
     __shared__ double lds[kEchoChunk][kEchoCols];
@@ -25,7 +26,7 @@ __global__ __launch_bounds__(max_threads_for_k(K)) void zwalk_kernel(const WalkA
                                   : (TAB == 3 ? kZFlippedEntries : (MFLAGS ? 8 * kZFlagStride / 16 : (NOFLUX ? 12 : 6)))];
     __shared__ uint4 small[6];
     __shared__ uint2 fix[TAB == 3 ? kZFlippedEntries : (MFLAGS ? 8 * kZFlagStride / 16 : 6)];
-    __shared__ uint32_t keys[TAB == 3 ? kZFlagKeyEntries / 4 : (TAB == 2 ? kZKeyEntries / 4 : 1)];
+    __shared__ __align__(16) uint32_t keys[TAB == 3 ? kZFlagKeyEntries / 4 : (TAB == 2 ? kZKeyEntries / 4 : 1)];
     __shared__ double ldelta[kMaxLabels];
     extern __shared__ uint32_t zlh[];   // EMODE 2, K == 1: per-label hit counts (blockDim x kLhStride)
     const uint64_t tile = tile_of_block(a);
@@ -33,7 +34,7 @@ __global__ __launch_bounds__(max_threads_for_k(K)) void zwalk_kernel(const WalkA
         return;  // spare workgroup of the XCD-striped grid (whole block leaves together)
     uint8_t *key_bytes = reinterpret_cast<uint8_t *>(keys);
     if (NOFLUX)
-        zbuild_table_noflux(a.zl, tab);
+        zbuild_table_noflux(a.zl, tab, SUB ? (uint32_t)a.shift : 0u);
     else if (TAB == 3)
         zbuild_table_flipped(a.zl, tab, fix);
     else if (MFLAGS)
@@ -51,7 +52,7 @@ __global__ __launch_bounds__(max_threads_for_k(K)) void zwalk_kernel(const WalkA
         zbuild_table_wide(small, tab);
         __syncthreads();
     }
-    zwalk_tile<EMODE, K, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, 1, false, ADISP, HITS>(
+    zwalk_tile<EMODE, K, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, 1, false, ADISP, HITS, SUB>(
         a, tile, a.partials ? a.partials + tile : nullptr, a.partial_stride, lds, tab, fix, ldelta, key_bytes,
         EMODE == 2 && K == 1 ? zlh : nullptr);
 }
@@ -90,19 +91,38 @@ static hipError_t launch_z(const WalkArgs &a, const LaunchShape &ls, uint32_t bl
     return hipGetLastError();
 }
 
+// Voxel division (a.shift > 0): one walker per lane, whatever ls.k says.
+template <int EMODE, bool WRAPFIX, bool NOFLUX, bool MFLAGS>
+static hipError_t launch_z_sub(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
+{
+    const size_t lh_bytes = EMODE == 2 ? (size_t)kLhStride * ls.threads * sizeof(uint32_t) : 0;
+    hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, 128, 2, NOFLUX, MFLAGS, false, true, true>), dim3(blocks),
+                       dim3(ls.threads), lh_bytes, st, a);
+    return hipGetLastError();
+}
+
 // a.zcache: 0 no chunk cache; 1 128-bit chunk with word select; 2 and 3 a
 // 128-bit chunk with the shift test and the direction drawn one step ahead,
 // through the byte-key table (2) or, for power-of-two periods, the wide
 // direction table (3; the 6-entry table otherwise); 4 the speculative CPMG
-// walk; 5 as 2 with a 64-bit (4 x 4 x 4 voxel) chunk, mirror walks with
+// and map walks; 5 as 2 with a 64-bit (4 x 4 x 4 voxel) chunk, mirror walks with
 // reflection flags (others run 2).
 template <int EMODE>
 hipError_t launch_z_mode(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
 {
-    // a.zcache 4: the speculative CPMG walk (one walker per lane); other
-    // modes and lane shapes take the pipelined chunk-cache walk
-    if (a.zcache == 4 && EMODE == 1 && ls.k == 1)
-        return launch_z_spec(a, ls, blocks, st);
+    // a.zcache 4: the speculative CPMG and map walks (one walker per lane);
+    // other modes and lane shapes take the pipelined chunk-cache walk
+    if (a.zcache == 4 && EMODE < 2 && (ls.k == 1 || a.shift))
+        return launch_z_spec(a, EMODE, ls, blocks, st);
+    if (a.shift) {
+        if (a.znoflux)
+            return launch_z_sub<EMODE, false, true, false>(a, ls, blocks, st);
+        if (a.zmflags)
+            return a.zl.wrapfix ? launch_z_sub<EMODE, true, false, true>(a, ls, blocks, st)
+                                : launch_z_sub<EMODE, false, false, true>(a, ls, blocks, st);
+        return a.zl.wrapfix ? launch_z_sub<EMODE, true, false, false>(a, ls, blocks, st)
+                            : launch_z_sub<EMODE, false, false, false>(a, ls, blocks, st);
+    }
     if (a.zcache == 4) {
         WalkArgs b = a;
         b.zcache = 2;
