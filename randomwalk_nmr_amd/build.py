@@ -18,8 +18,9 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = "gfx950"
 
-# the slowest to compile first
-HIP_SOURCES = ["zwalk_cpmg.hip", "zwalk_labels.hip", "zwalk_map.hip", "zwalk_kernels.hip", "zwalk_spec.hip",
+# the slowest to compile first; "file:m" compiles file for energy mode m
+HIP_SOURCES = ["zwalk_mirror.hip:1", "zwalk_labels.hip", "zwalk_mirror.hip:2", "zwalk_cpmg.hip", "zwalk_mirror.hip:0",
+               "zwalk_kernels.hip", "zwalk_map.hip", "zwalk_spec.hip",
                "batch_kernels.hip", "walk_kernels.hip", "backward_kernels.hip", "locality_kernels.hip", "capi.hip",
                "drivers.hip", "probe_kernels.hip"]
 CXX_SOURCES = ["laplace.cpp", "host_sim.cpp", "image_io.cpp", "histogram.cpp", "config.cpp", "output.cpp"]
@@ -82,12 +83,14 @@ def build(verbose: bool = False, jobs: int = 0) -> str:
     if verbose and load_flags:
         print("indexed buffer load unavailable: building the raw-load form")
     cmds, objs = [], []
-    for src in HIP_SOURCES:
+    for entry in HIP_SOURCES:
+        src, _, mode = entry.partition(":")
         path = os.path.join(CSRC, src)
         if not os.path.exists(path):
             continue
-        obj = os.path.join(OUT_DIR, src + ".o")
-        cmds.append([HIPCC, *HIP_FLAGS, *load_flags, "-c", path, "-o", obj])
+        obj = os.path.join(OUT_DIR, src + mode + ".o")
+        mode_flags = [f"-DRWNMR_MIRROR_EMODE={mode}"] if mode else []
+        cmds.append([HIPCC, *HIP_FLAGS, *load_flags, *mode_flags, "-c", path, "-o", obj])
         objs.append(obj)
     for src in CXX_SOURCES:
         path = os.path.join(CSRC, src)

@@ -109,7 +109,7 @@ struct rwnmr_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     LaunchShape shape{256, 1};
-    // no shape / no image form was asked for: run_shape and attach_zimage choose by the run
+    // no shape / no image form was asked for: plan_run and attach_zimage choose by the run
     bool shape_auto = true, form_auto = true;
     // walker staging for host-pointer calls
     DevBuf x, y, z, seed, energy, hits, penalty, x0, y0, z0;
@@ -145,6 +145,7 @@ struct rwnmr_ctx {
     // locality ordering: Morton-sorted walkers, XCD-striped tiles, re-sorted
     // every resort_every echoes (only for runs of at least min_walkers)
     int locality = 1;
+    bool locality_auto = true;   // not asked for: runs too short to gain by it stay unsorted (sorts_pay)
     uint32_t resort_every = 1000;
     uint64_t locality_min_walkers = 65536;
     DevBuf lkeys, lidx, lsort_tmp;
@@ -554,16 +555,52 @@ void attach_zimage(rwnmr_ctx *c, const rwnmr_image *img, int bc, int emode, Walk
     }
 }
 
-// Launch shape of a CPMG or map run (a as attach_zimage left it): the
-// context's, or, where none was set, 64-thread blocks for a speculative walk
-// that leaves a SIMD of each CU free, so that its waves spread over as many
-// CUs as there are (128^3, 30k walkers: 152 ns per step against 176 with 256
-// threads; 65,536 walkers: 178 against 167).
-LaunchShape run_shape(const rwnmr_ctx *c, const WalkArgs &a, int emode)
+// Whether a run of `steps` steps gains by the position ordering of its
+// walkers.  A sort with its gather and scatter costs 110 us at 200k walkers
+// and 250 us at 1M; the sorted walk is 0-4% faster at 100k-300k walkers (12%
+// on a 256^3 mirror image) and 12-18% at 1M, so the line lies at about 2 ms
+// of walk, at 0.8 ns per 1000 walkers and step (at least 200 ns per step).
+bool sorts_pay(uint64_t n, uint64_t steps)
 {
-    return c->shape_auto && a.zwords && a.zcache == 4 && emode < 2 && a.n <= kSpecMaxWalkers / 4 * 3
-               ? LaunchShape{64u, 1u}
-               : c->shape;
+    return (double)steps * std::max(200.0, 0.8e-3 * (double)n) >= 2.0e6;
+}
+
+// Launch shape of a CPMG, map or per-label run (a as attach_zimage left it)
+// and, where no image form was asked for, the form of a chunk-cache walk.
+// `sorted`: the walkers are kept in position order.
+//  - The speculative walk runs in 64-thread blocks while it leaves a SIMD of
+//    each CU free, so that its waves spread over as many CUs as there are
+//    (128^3, 30k walkers: 152 ns per step against 176 with 256 threads;
+//    65,536 walkers: 178 against 167).
+//  - The 8-byte chunk (form 6) saves 3 instructions per step and costs a
+//    quarter more chunk loads, which pays where these hit the L2: where the
+//    part of the image that is read fits the 4 MiB of one XCD, 3-9% faster up
+//    to 300k walkers and, sorted, at 1M (256^3 mirror, 3 steps per echo: 789
+//    against 855 ns per step), but slower for 1M unsorted ones (1071 against
+//    985) and on a 512^3 mirror image (16 MiB; 1M sorted: 5% slower).
+//  - Sorted mirror walks of a whole round of resident 1024-thread blocks
+//    (512 of them) take the flag-keyed tables of that block size (1M walkers,
+//    12 steps per echo: 746 against 873 ns per step with 256 threads; 300k:
+//    350 against 283).
+constexpr uint64_t kChunk8Unsorted = 400000;
+constexpr uint32_t kChunk8ImageBits = 25;   // log2 of the addresses of 4 MiB
+
+LaunchShape plan_run(const rwnmr_ctx *c, WalkArgs &a, int emode, bool sorted)
+{
+    LaunchShape ls = c->shape;
+    if (c->shape_auto && a.zwords && emode < 2) {
+        if (a.zcache == 4 && a.n <= kSpecMaxWalkers / 4 * 3)
+            ls = LaunchShape{64u, 1u};
+        else if (sorted && a.zmflags && a.n >= (uint64_t)c->balanced_slots * 1024u && c->balanced_slots)
+            ls = LaunchShape{1024u, 1u};
+    }
+    if (c->form_auto && a.zwords && a.zcache == 2 && (ls.k == 1 || a.shift)) {
+        // addresses of the base image, of its first octant with reflection flags
+        const uint32_t read_bits = a.zl.bits - 3u * (uint32_t)a.shift - (a.zmflags ? 3u : 0u);
+        if (read_bits <= kChunk8ImageBits && (sorted || a.n <= kChunk8Unsorted))
+            a.zcache = 5;
+    }
+    return ls;
 }
 
 hipError_t launch_any_walk(const WalkArgs &a, int bc, int emode, const LaunchShape &ls, hipStream_t st)
@@ -810,8 +847,10 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
     attach_zimage(c, img, bc, emode, a, true, true);
     if (jac && (!a.zwords || !a.zlabels))
         return fail(c, RWNMR_ERR_INVALID, "Jacobian forward: needs the unfolded labelled image");
+    const bool local = emode < 2 && shift == 0 && c->locality && w->n >= c->locality_min_walkers &&
+                       (!c->locality_auto || sorts_pay(w->n, (uint64_t)echoes * steps_per_echo));
     // the Jacobian forward holds one walker per lane
-    const LaunchShape shape = jac ? LaunchShape{c->shape.threads, 1u} : run_shape(c, a, emode);
+    const LaunchShape shape = jac ? LaunchShape{c->shape.threads, 1u} : plan_run(c, a, emode, local);
     // tiles, one echo-partial column each (balanced tiles where they apply)
     const uint32_t blocks = jac ? rwnmr::walk_grid_blocks(w->n, shape, (int)shift) : walk_columns(c, a, emode, shape);
     a.partial_stride = blocks;
@@ -845,7 +884,6 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
             jrows = c->jac_rows.as<double>();
         }
     }
-    const bool local = emode < 2 && shift == 0 && c->locality && w->n >= c->locality_min_walkers;
     if (local) {
         a.steps_per_echo = steps_per_echo;
         if ((s = walk_local(c, img, a, bc, emode, echoes, steps_per_echo, echo_sums ? sums : nullptr, chunk,
@@ -1015,6 +1053,7 @@ rwnmr_status rwnmr_ctx_set_locality(rwnmr_ctx *c, int32_t enable, uint32_t resor
     if (!c)
         return RWNMR_ERR_INVALID;
     c->locality = enable != 0;
+    c->locality_auto = false;
     c->resort_every = resort_every ? resort_every : 1000;
     c->locality_min_walkers = min_walkers;
     return RWNMR_OK;
@@ -1243,12 +1282,13 @@ rwnmr_status rwnmr_map_run(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *
     a.energy = nullptr;  // the map walk never touches energies
     a.echoes = 1;
     attach_zimage(c, img, bc, 0, a, true, true);
+    const LaunchShape shape = plan_run(c, a, 0, false);
     uint64_t left = steps;
     while (left > 0) {
         const uint32_t now = (uint32_t)std::min<uint64_t>(left, 1ull << 30);
         a.steps_per_echo = now;
         hipEvent_t t0 = timing_begin(c);
-        RW_HIP(c, launch_any_walk(a, bc, 0, run_shape(c, a, 0), c->stream));
+        RW_HIP(c, launch_any_walk(a, bc, 0, shape, c->stream));
         timing_end(c, t0);
         left -= now;
     }
@@ -1297,10 +1337,11 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
     const LaunchShape saved = c->shape;
     const int saved_unfolded = c->unfolded;
     const uint32_t saved_resort = c->resort_every;
-    const bool saved_form_auto = c->form_auto, saved_shape_auto = c->shape_auto;
+    const bool saved_form_auto = c->form_auto, saved_shape_auto = c->shape_auto, saved_locality_auto = c->locality_auto;
     auto restore = [&]() {
         c->form_auto = saved_form_auto;
         c->shape_auto = saved_shape_auto;
+        c->locality_auto = saved_locality_auto;
         c->timing = was_timing;
         c->kernel_ms = saved_ms;
         c->kernel_launches = saved_launches;
@@ -1310,7 +1351,8 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
         cleanup();
     };
     c->timing = true;
-    c->form_auto = c->shape_auto = false;   // each trial runs the shape and form it is set to
+    // each trial runs the shape, form and ordering it is set to
+    c->form_auto = c->shape_auto = c->locality_auto = false;
     (void)hipStreamSynchronize(c->stream);
     timing_collect(c);
     // One trial run from the caller's start state; returns the walk kernels'
@@ -1528,7 +1570,7 @@ rwnmr_status rwnmr_cpmg_run_noalloc(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_
     a.n_labels = img->n_labels;
     // an unfolded image is used only when an earlier call built it
     attach_zimage(c, img, bc, 1, a, true, true, false);
-    const LaunchShape shape = run_shape(c, a, 1);
+    const LaunchShape shape = plan_run(c, a, 1, false);
     const uint32_t blocks = rwnmr::walk_grid_blocks(w->n, shape, (int)shift);
     // echoes per launch: rows 0..chunk of [echo][block] partials must fit the scratch
     uint64_t chunk = echoes ? echoes : 1;
@@ -1622,7 +1664,7 @@ rwnmr_status rwnmr_cpmg_graph_create(rwnmr_ctx *c, const rwnmr_image *img, rwnmr
     WalkArgs a = base_args(img, v, w, 0, c->flag.as<uint32_t>());
     a.n_labels = img->n_labels;
     attach_zimage(c, img, bc, 1, a, true, true, true);
-    const LaunchShape shape = run_shape(c, a, 1);
+    const LaunchShape shape = plan_run(c, a, 1, false);
     const uint32_t blocks = rwnmr::walk_grid_blocks(n, shape, 0);
     uint64_t chunk = echoes ? echoes : 1;
     if (echo_sums && blocks)

@@ -506,12 +506,11 @@ __device__ __forceinline__ uint32_t zcompact(uint32_t v, uint32_t m)
 // to a.jac_partials + tile, row stride part_stride, label stride (a.echoes +
 // 1) part_stride, through the 8-value reduce-scatter (lds8: the staging of
 // stage_echo_sets8).
-// ADISP (mirror walks with reflection flags, every period above 2 kZFlush:
-// zaddress_displacement_ok): no packed displacement per move; each flush
-// recovers the walker's unbounded moves from its address change since the
-// last flush (per axis, the coordinate change taken modulo the period into
-// (-period / 2, period / 2), negated along reflected axes), one VALU per
-// move fewer.
+// ADISP (one walker per lane, periodic and mirror, every period at least
+// kZMinDispPeriod: zaddress_displacement_ok): no packed displacement per
+// move; each flush recovers the walker's unbounded moves from the change of
+// its address coordinates since the last one (modulo the period into (-period
+// / 2, period / 2), negated along reflected axes).
 // SUB: voxel division by 2^a.shift (one walker per lane): a.zl addresses
 // sub-voxels, interleaved like the image's voxels above the low 3 a.shift
 // bits, so the voxel address is a shift of the sub-voxel one (1 VALU per
@@ -531,9 +530,9 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     static_assert(!NOFLUX || CACHE >= 64, "noflux: pipelined chunk-cache walk only");
     static_assert(TAB != 3 || (MFLAGS && CACHE >= 64), "flag-keyed tables: pipelined mirror walk only");
     static_assert(NS == 1 || (NS == 8 && EMODE == 2 && K == 1 && CACHE >= 64), "label sets: 8 sets, K == 1");
-    static_assert(!ADISP || (MFLAGS && !NOFLUX && CACHE >= 64), "address displacements: pipelined mirror walk");
-    static_assert(HITS || (EMODE == 1 && CACHE >= 64), "uncounted hits: pipelined CPMG walk");
-    static_assert(!SUB || (CACHE == 128 && K == 1), "voxel division: pipelined walk of one walker per lane");
+    static_assert(!ADISP || (K == 1 && !NOFLUX && CACHE >= 64), "address displacements: pipelined, one walker per lane");
+    static_assert(HITS || (EMODE >= 1 && CACHE >= 64), "uncounted hits: pipelined CPMG and per-label walks");
+    static_assert(!SUB || (CACHE >= 64 && K == 1), "voxel division: pipelined walk of one walker per lane");
     const uint32_t sub = SUB ? (uint32_t)a.shift : 0u, sub3 = 3u * sub;
     auto voxel = [&](uint32_t c) { return SUB ? c >> sub3 : c; };
     // label-set walks count no per-label hits (a.label_hits is null)
@@ -541,7 +540,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     constexpr int NL = (EMODE == 2 && !LH_LDS && NS == 1) ? kMaxLabels : 1;
     const char *words = reinterpret_cast<const char *>(a.zwords);
     const zrsrc_t zrsrc =
-        CACHE == 64 ? zchunk_rsrc8(a.zwords, a.zl.bits) : zchunk_rsrc(a.zwords, a.zl.bits - sub3);
+        CACHE == 64 ? zchunk_rsrc8(a.zwords, a.zl.bits - sub3) : zchunk_rsrc(a.zwords, a.zl.bits - sub3);
     // the tile's walkers: blockDim x K from tile x blockDim x K, or with
     // balanced tiles a.tile_walkers (at most blockDim, K == 1) from tile x
     // a.tile_walkers
@@ -553,7 +552,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     const int n_labels = a.n_labels;
 
     uint32_t A[K], C[K], Hc[K];
-    uint32_t A0[K];   // ADISP: the address at the last flush
+    int32_t AC[3];    // ADISP: the address coordinates at the last flush
     uint32_t FO[K];   // MFLAGS: the walker's direction table offset (flags x kZFlagStride)
     uint32_t QB[K];   // chunk cache: chunk id (address >> 6 or >> 7) held in QV
     uint4 QV[K];
@@ -603,7 +602,9 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
             FO[k] = 0u;
         }
         P[k] = 0;
-        A0[k] = A[k];
+        if (ADISP)
+            for (int ax = 0; ax < 3; ++ax)
+                AC[ax] = (int32_t)zcompact(A[k], a.zl.m[ax]);
         PW[k] = 0u;
         PEND[k] = false;
         if (NS > 1)
@@ -638,12 +639,14 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
                 dy = (int32_t)zcompact(A[k], a.zl.m[1]) - Y[k];
                 dz = (int32_t)zcompact(A[k], a.zl.m[2]) - Z[k];
             } else if constexpr (ADISP) {
-                const uint32_t flags = FO[k] / (TAB == 3 ? kZKeyEntries : kZFlagStride);
+                const uint32_t flags = MFLAGS ? FO[k] / (TAB == 3 ? kZKeyEntries : kZFlagStride) : 0u;
                 int32_t d[3];
 #pragma unroll
                 for (int ax = 0; ax < 3; ++ax) {
                     const int32_t per = (int32_t)a.zl.period[ax];
-                    int32_t s = (int32_t)zcompact(A[k], a.zl.m[ax]) - (int32_t)zcompact(A0[k], a.zl.m[ax]);
+                    const int32_t now = (int32_t)zcompact(A[k], a.zl.m[ax]);
+                    int32_t s = now - AC[ax];
+                    AC[ax] = now;
                     if (s > per / 2)
                         s -= per;
                     else if (s < -(per / 2))
@@ -653,7 +656,6 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
                 dx = d[0];
                 dy = d[1];
                 dz = d[2];
-                A0[k] = A[k];
             } else {
                 zunpack(P[k], dx, dy, dz);
                 P[k] = 0;
@@ -739,7 +741,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
                 if (CACHE == 128)
                     zchunk_fill_buf(zrsrc, voxel(C[k]), QB[k], QV[k]);
                 else
-                    zchunk_fill_buf8(zrsrc, C[k], QB[k], QV[k]);
+                    zchunk_fill_buf8(zrsrc, voxel(C[k]), QB[k], QV[k]);
             });
             static_for<K>([&](auto kc) {
                 constexpr int k = decltype(kc)::value;
@@ -766,7 +768,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
         static_for<K>([&](auto kc) {
             constexpr int k = decltype(kc)::value;
             const uint32_t wall = wallv[k];
-            if (CACHE >= 64 && DISP && EMODE == 1) {
+            if (CACHE >= 64 && EMODE == 1 && DISP) {
                 // a packed displacement to keep as well: two short divergent
                 // paths (3-5% faster than masks from 5 waves per SIMD on)
                 if (__builtin_expect(wall != 0u, 0)) {
@@ -776,6 +778,21 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
                 } else {
                     A[k] = C[k];
                     P[k] += DP[k];
+                }
+                return;
+            }
+            if (CACHE >= 64 && EMODE == 1 && TAB == 3) {
+                // whole rounds of 8 waves per SIMD: divergent paths as well
+                // (512^3, 1M walkers: 1.0% faster than masks; the empty asm
+                // keeps the compiler from turning the paths into selects)
+                if (__builtin_expect(wall != 0u, 0)) {
+                    if (HITS)
+                        Hc[k] += 1u;
+                    asm volatile("" : "+v"(E[k]));
+                    E[k] *= DL[k];
+                } else {
+                    asm volatile("" : "+v"(A[k]));
+                    A[k] = C[k];
                 }
                 return;
             }
@@ -816,11 +833,12 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
     };
 
     const uint64_t set_stride = (uint64_t)(echoes + 1) * part_stride;
+    const uint32_t flush_every = ADISP ? zflush_interval(a.zl) : kZFlush;
     uint32_t since = 0;
     auto walk_echo = [&]() {
         uint32_t left = spe;
         while (left) {
-            const uint32_t ns = NOFLUX || left < kZFlush - since ? left : kZFlush - since;
+            const uint32_t ns = NOFLUX || left < flush_every - since ? left : flush_every - since;
             // two steps per trip: the pipelined direction entry then lives in
             // alternating registers instead of being copied every step
             uint32_t i = 0;
@@ -832,7 +850,7 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
                 step();
             since += ns;
             left -= ns;
-            if (!NOFLUX && since == kZFlush) {
+            if (!NOFLUX && since == flush_every) {
                 flush();
                 since = 0;
             }

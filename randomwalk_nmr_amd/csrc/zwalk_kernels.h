@@ -13,13 +13,26 @@ namespace rwnmr {
 // component must stay within +-511).
 static constexpr uint32_t kZFlush = 511;
 
-// Address displacements recover the unbounded moves when every period of
-// the layout exceeds twice the flush interval: a walker moves at most
-// kZFlush voxels per axis between flushes, less than half a period, so the
-// coordinate change modulo the period is the move itself.
+// Address displacements: the walk keeps no displacement but takes its
+// unbounded moves from the change of its address coordinates, every
+// zflush_interval steps.  A walker moves at most that many voxels per axis
+// between two flushes, less than half of every period, so the coordinate
+// change modulo the period is the move itself.  A flush costs about 70
+// instructions, a packed displacement 2 per step, so it pays from periods of
+// 128 (63 steps) on.
+static constexpr uint32_t kZMinDispPeriod = 128;
+
+__host__ __device__ inline uint32_t zmin_period(const ZLayout &zl)
+{
+    const uint32_t p = zl.period[0] < zl.period[1] ? zl.period[0] : zl.period[1];
+    return p < zl.period[2] ? p : zl.period[2];
+}
+
+__host__ __device__ inline uint32_t zflush_interval(const ZLayout &zl) { return (zmin_period(zl) - 1u) / 2u; }
+
 __host__ __device__ inline bool zaddress_displacement_ok(const ZLayout &zl)
 {
-    return zl.period[0] > 2u * kZFlush && zl.period[1] > 2u * kZFlush && zl.period[2] > 2u * kZFlush;
+    return zmin_period(zl) >= kZMinDispPeriod;
 }
 
 // True when a CPMG launch of shape ls runs the mirror walk with flag-keyed

@@ -19,7 +19,12 @@ hipError_t launch_z_spec(const WalkArgs &a, int emode, const LaunchShape &ls, ui
 
 template <int EMODE, int K, bool WRAPFIX, int CACHE, int TAB, bool NOFLUX = false, bool MFLAGS = false,
           bool ADISP = false, bool HITS = true, bool SUB = false>
-__global__ __launch_bounds__(max_threads_for_k(K)) void zwalk_kernel(const WalkArgs a)
+// 80 SGPRs: with 16 more kept for the trap handler a wave then takes 96 of the
+// SIMD's 800, so 8 waves fit; with 82 it takes 112, and of two 1024-thread
+// blocks per CU only one is resident (512^3 walk: 1.07e12 against 1.25e12
+// walker-steps/s).
+__global__ __launch_bounds__(max_threads_for_k(K)) __attribute__((amdgpu_num_sgpr(80))) void zwalk_kernel(
+    const WalkArgs a)
 {
     __shared__ double lds[kEchoChunk][kEchoCols];
     __shared__ uint4 tab[TAB == 1 ? kZWideEntries
@@ -57,25 +62,29 @@ __global__ __launch_bounds__(max_threads_for_k(K)) void zwalk_kernel(const WalkA
         EMODE == 2 && K == 1 ? zlh : nullptr);
 }
 
-template <int EMODE, bool WRAPFIX, int CACHE, int TAB, bool NOFLUX = false, bool MFLAGS = false>
+// ONE: ls.k is 1, and only that instance is built.
+template <int EMODE, bool WRAPFIX, int CACHE, int TAB, bool NOFLUX = false, bool MFLAGS = false, bool ONE = false>
 static hipError_t launch_z(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
 {
-    // mirror CPMG of one walker per lane on images whose periods all exceed
-    // twice the flush interval: unbounded moves from address displacements
-    if constexpr (EMODE == 1 && MFLAGS && TAB == 3 && !NOFLUX) {
+    // EMODE 2 with one walker per lane keeps the per-label hit counts in LDS
+    const size_t lh_bytes = EMODE == 2 ? (size_t)kLhStride * ls.threads * sizeof(uint32_t) : 0;
+    // one walker per lane on images of periods of 128 and more: unbounded
+    // moves from address displacements; hits counted only when asked for
+    if constexpr (CACHE >= 64 && TAB >= 2 && !NOFLUX) {
         if (ls.k == 1 && zaddress_displacement_ok(a.zl)) {
-            // hit counts only when the caller asked for them
-            if (a.hits)
+            if (EMODE == 0 || a.hits)
                 hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, true>), dim3(blocks),
-                                   dim3(ls.threads), 0, st, a);
+                                   dim3(ls.threads), lh_bytes, st, a);
             else
-                hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, true, false>),
-                                   dim3(blocks), dim3(ls.threads), 0, st, a);
+                hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, true, EMODE == 0>),
+                                   dim3(blocks), dim3(ls.threads), lh_bytes, st, a);
             return hipGetLastError();
         }
     }
-    // EMODE 2 with one walker per lane keeps the per-label hit counts in LDS
-    const size_t lh_bytes = EMODE == 2 ? (size_t)kLhStride * ls.threads * sizeof(uint32_t) : 0;
+    if constexpr (ONE) {
+        hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS>), dim3(blocks), dim3(ls.threads), lh_bytes, st, a);
+        return hipGetLastError();
+    }
     switch (ls.k) {
     case 1: hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS>), dim3(blocks), dim3(ls.threads), lh_bytes, st, a); break;
     case 2: hipLaunchKernelGGL((zwalk_kernel<EMODE, 2, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS>), dim3(blocks), dim3(ls.threads), 0, st, a); break;
@@ -91,22 +100,32 @@ static hipError_t launch_z(const WalkArgs &a, const LaunchShape &ls, uint32_t bl
     return hipGetLastError();
 }
 
-// Voxel division (a.shift > 0): one walker per lane, whatever ls.k says.
+// Voxel division (a.shift > 0): one walker per lane, whatever ls.k says, and
+// the 8-byte chunk, which a sub-voxel step leaves less often.
 template <int EMODE, bool WRAPFIX, bool NOFLUX, bool MFLAGS>
 static hipError_t launch_z_sub(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
 {
     const size_t lh_bytes = EMODE == 2 ? (size_t)kLhStride * ls.threads * sizeof(uint32_t) : 0;
-    hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, 128, 2, NOFLUX, MFLAGS, false, true, true>), dim3(blocks),
-                       dim3(ls.threads), lh_bytes, st, a);
+    if (!NOFLUX && zaddress_displacement_ok(a.zl))
+        hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, 64, 2, NOFLUX, MFLAGS, !NOFLUX, true, true>),
+                           dim3(blocks), dim3(ls.threads), lh_bytes, st, a);
+    else
+        hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, 64, 2, NOFLUX, MFLAGS, false, true, true>), dim3(blocks),
+                           dim3(ls.threads), lh_bytes, st, a);
     return hipGetLastError();
 }
+
+// Mirror walks with reflection flags (a.zmflags, a.zcache >= 2), instantiated
+// apart from the rest (zwalk_mirror.hip): they are the larger half to compile.
+template <int EMODE>
+hipError_t launch_z_mirror(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st);
 
 // a.zcache: 0 no chunk cache; 1 128-bit chunk with word select; 2 and 3 a
 // 128-bit chunk with the shift test and the direction drawn one step ahead,
 // through the byte-key table (2) or, for power-of-two periods, the wide
 // direction table (3; the 6-entry table otherwise); 4 the speculative CPMG
 // and map walks; 5 as 2 with a 64-bit (4 x 4 x 4 voxel) chunk, mirror walks with
-// reflection flags (others run 2).
+// reflection flags and other walks of one walker per lane (the rest run 2).
 template <int EMODE>
 hipError_t launch_z_mode(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
 {
@@ -128,28 +147,20 @@ hipError_t launch_z_mode(const WalkArgs &a, const LaunchShape &ls, uint32_t bloc
         b.zcache = 2;
         return launch_z_mode<EMODE>(b, ls, blocks, st);
     }
+    if (a.zcache == 5 && ls.k == 1 && !a.zmflags) {   // noflux and periodic, 8-byte chunk cache
+        if (a.znoflux)
+            return launch_z<EMODE, false, 64, 2, true, false, true>(a, ls, blocks, st);
+        return a.zl.wrapfix ? launch_z<EMODE, true, 64, 2, false, false, true>(a, ls, blocks, st)
+                            : launch_z<EMODE, false, 64, 2, false, false, true>(a, ls, blocks, st);
+    }
     if (a.znoflux)   // noflux on the periodic image: pipelined byte-key walk only
         return a.zcache >= 2 ? launch_z<EMODE, false, 128, 2, true>(a, ls, blocks, st) : hipErrorInvalidValue;
-    if (a.zmflags && a.zcache == 5) {   // mirror, 8-byte chunk cache
-        if (EMODE < 2 && ls.threads >= 1024)
-            return a.zl.wrapfix ? launch_z<EMODE, true, 64, 3, false, true>(a, ls, blocks, st)
-                                : launch_z<EMODE, false, 64, 3, false, true>(a, ls, blocks, st);
-        return a.zl.wrapfix ? launch_z<EMODE, true, 64, 2, false, true>(a, ls, blocks, st)
-                            : launch_z<EMODE, false, 64, 2, false, true>(a, ls, blocks, st);
-    }
+    if (a.zmflags && a.zcache >= 2)   // mirror, walkers folded to the first octant with reflection flags
+        return launch_z_mirror<EMODE>(a, ls, blocks, st);
     if (a.zcache == 5) {
         WalkArgs b = a;
         b.zcache = 2;
         return launch_z_mode<EMODE>(b, ls, blocks, st);
-    }
-    if (a.zmflags && a.zcache >= 2) {   // mirror, walkers folded to the first octant with reflection flags
-        // CPMG and map walks of 1024-thread blocks read the flag-keyed
-        // tables (58 KiB of LDS: two blocks per CU, 8 waves per SIMD)
-        if (EMODE < 2 && ls.threads >= 1024)
-            return a.zl.wrapfix ? launch_z<EMODE, true, 128, 3, false, true>(a, ls, blocks, st)
-                                : launch_z<EMODE, false, 128, 3, false, true>(a, ls, blocks, st);
-        return a.zl.wrapfix ? launch_z<EMODE, true, 128, 2, false, true>(a, ls, blocks, st)
-                            : launch_z<EMODE, false, 128, 2, false, true>(a, ls, blocks, st);
     }
     if (a.zl.wrapfix) {
         switch (a.zcache) {
