@@ -565,6 +565,39 @@ bool sorts_pay(uint64_t n, uint64_t steps)
     return (double)steps * std::max(200.0, 0.8e-3 * (double)n) >= 2.0e6;
 }
 
+// Whether a field walk of `steps` steps gains by lanes in position order: the
+// field has to spill an XCD's 4 MiB L2 (64^3, 2 MiB: 1153 against 1144 us for
+// 1600 steps of 100k walkers), and the sort, 45 us, has to be earned (100x90x80
+// and 150x120x101, 256 steps of 70k-100k walkers: 311-350 against 268-298 us;
+// 32 steps: 76-82 against 114-119; 256^3, 300k walkers, 1600 steps: 9264
+// against 6619).
+bool field_order_pays(const rwnmr_image *img, uint64_t steps)
+{
+    const uint64_t voxels = (uint64_t)img->W * (uint64_t)img->H * (uint64_t)img->D;
+    return steps >= 256 && 8 * voxels > (4ull << 20);
+}
+
+// Sorts the walkers' indices by the Morton code of their image block; a.order
+// is where a field walk's lanes find them.
+rwnmr_status order_by_position(rwnmr_ctx *c, const rwnmr_image *img, WalkArgs &a, int bc)
+{
+    const uint64_t n = a.n;
+    const uint32_t side = (uint32_t)std::max(img->W, std::max(img->H, img->D));
+    int key_bits = 3;
+    while (key_bits < 30 && (4u << (key_bits / 3)) < side)
+        key_bits += 3;
+    size_t tmp_bytes = 0;
+    RW_HIP(c, rwnmr::sort_pairs_temp_bytes(n, key_bits, &tmp_bytes));
+    RW_HIP(c, c->lsort_tmp.reserve(tmp_bytes + 256));
+    RW_HIP(c, c->lkeys.reserve(8 * n));
+    RW_HIP(c, c->lidx.reserve(8 * n));
+    uint32_t *keys = c->lkeys.as<uint32_t>(), *idx = c->lidx.as<uint32_t>();
+    RW_HIP(c, rwnmr::launch_morton_keys(bc, a.x, a.y, a.z, n, img->W, img->H, img->D, keys, idx, c->stream));
+    RW_HIP(c, rwnmr::sort_pairs(c->lsort_tmp.p, tmp_bytes, keys, keys + n, idx, idx + n, n, key_bits, c->stream));
+    a.order = idx + n;
+    return RWNMR_OK;
+}
+
 // Launch shape of a CPMG, map or per-label run (a as attach_zimage left it)
 // and, where no image form was asked for, the form of a chunk-cache walk.
 // `sorted`: the walkers are kept in position order.
@@ -906,9 +939,16 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
         a.tile_map = 1;
         a.n_tiles = blocks;
     }
+    // field walks in position order
+    const bool ordered = emode == 3 && c->locality && w->n >= c->locality_min_walkers && w->n <= 0xFFFFFFFFull &&
+                         (!c->locality_auto || field_order_pays(img, (uint64_t)echoes * steps_per_echo));
+    if (ordered)
+        chunk = std::min<uint64_t>(chunk, std::max<uint32_t>(1u, c->resort_every));
     uint32_t done = 0;
     do {
         const uint32_t ne = (uint32_t)std::min<uint64_t>(chunk, (uint64_t)echoes - done);
+        if (ordered && (s = order_by_position(c, img, a, bc)) != RWNMR_OK)
+            return s;
         a.echoes = ne;
         a.partials = echo_sums ? c->partials.as<double>() : nullptr;
         a.jac_partials = jac ? c->jac_partials.as<double>() : nullptr;

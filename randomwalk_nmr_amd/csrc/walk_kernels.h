@@ -61,6 +61,7 @@ struct WalkArgs {
     const double *field;
     double gammatau;
     double *p_alive, *phase;
+    const uint32_t *order;   // nullable: lane i walks walker order[i]
 };
 
 struct LaunchShape {
