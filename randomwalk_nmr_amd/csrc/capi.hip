@@ -55,6 +55,52 @@ struct DevBuf {
     template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
+// Host-pointer calls copy a handful of small arrays each way, and a copy from or
+// to pageable memory costs 8-15 us however small it is: up to kPackedBytes the
+// arrays travel as one pinned block, results first, penalty last.  A host CPMG
+// call of 2 steps: 2,000 walkers 75 us (224 array by array), 30,000 153 (247),
+// 100,000 346 (479); 200,000 (7 MB) 1525 (813), so the line lies at 4 MiB.
+constexpr size_t kPackedBytes = 4u << 20;
+
+struct PackedLayout {
+    size_t x = 0, y = 0, z = 0, seed = 0, energy = 0, hits = 0, penalty = 0;   // byte offsets, multiples of 256
+    size_t results = 0, total = 0;
+};
+
+// Pinned host buffer of at most kPackedBytes and some room for results.
+struct PinnedBuf {
+    char *p = nullptr;
+    size_t bytes = 0;
+    // false when the host has no pinned memory to give (the caller copies directly)
+    bool reserve(size_t want)
+    {
+        if (want <= bytes)
+            return true;
+        release();
+        if (hipHostMalloc((void **)&p, want, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        bytes = want;
+        return true;
+    }
+    void release()
+    {
+        if (p)
+            (void)hipHostFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
+};
+
+// A result waiting in pinned memory for its caller's array.
+struct HostResult {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+
 __global__ void fill_u32_kernel(uint32_t *p, uint32_t v, uint64_t n)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -116,6 +162,16 @@ struct rwnmr_ctx {
     // per-call small arrays and reductions
     DevBuf partials, sums, label_delta, label_hits, steps_inc, kvec, set_delta;
     DevBuf jac_partials, jac_rows;   // Jacobian forward: per-label partials and host-call rows
+    // host-pointer calls of up to kPackedBytes: walker arrays and results pass
+    // through one pinned buffer and one device buffer (stage_in, host_out)
+    PinnedBuf pinned;
+    DevBuf packed;
+    bool staging_open = false;    // `pinned` may be read or written by work on the stream
+    bool packed_in = false;       // this call's walkers are in `packed`
+    size_t pinned_used = 0;       // bytes of `pinned` taken by this call
+    PackedLayout packed_at;       // ... laid out so
+    HostResult results[16];       // copies to make once the stream is drained
+    int n_results = 0;
     // internal-field CPMG staging (host-pointer calls)
     DevBuf field, p_alive, phase;
     DevBuf msamples;   // PFGSE per-sample sums (host-pointer calls)
@@ -191,10 +247,19 @@ namespace {
 
 rwnmr_status fail(rwnmr_ctx *c, rwnmr_status code, const std::string &msg)
 {
-    if (c)
+    if (c) {
         c->err = msg;
+        c->n_results = 0;   // the failed call's arrays may be gone by the next synchronisation
+    }
     return code;
 }
+
+#define RW_ST(call)                                                                                         \
+    do {                                                                                                    \
+        const rwnmr_status st_ = (call);                                                                    \
+        if (st_ != RWNMR_OK)                                                                                \
+            return st_;                                                                                     \
+    } while (0)
 
 #define RW_HIP(ctx, call)                                                                                   \
     do {                                                                                                    \
@@ -273,6 +338,10 @@ rwnmr_status sync_and_check(rwnmr_ctx *c)
     if (scratch_flag)
         RW_HIP(c, hipMemcpyAsync(c->host_flag + 1, c->scratch, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     RW_HIP(c, hipStreamSynchronize(c->stream));
+    for (int i = 0; i < c->n_results; ++i)
+        memcpy(c->results[i].dst, c->results[i].src, c->results[i].bytes);
+    c->n_results = 0;
+    c->staging_open = c->packed_in = false;
     c->scratch_flag_pending = false;
     timing_collect(c);
     if (c->host_flag[0] || c->host_flag[1])
@@ -325,6 +394,43 @@ struct WalkerView {
     const double *penalty;
 };
 
+PackedLayout packed_layout(const rwnmr_walkers *w)
+{
+    PackedLayout L;
+    const size_t n = w->n > kPackedBytes ? kPackedBytes : (size_t)w->n;   // no overflow; too large either way
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) / 256 * 256;
+        return o;
+    };
+    L.x = take(4 * n);
+    L.y = take(4 * n);
+    L.z = take(4 * n);
+    L.seed = take(8 * n);
+    L.energy = take(w->energy ? 8 * n : 0);
+    L.hits = take(w->hits ? 4 * n : 0);
+    L.results = at;
+    L.penalty = take(w->penalty ? 8 * n : 0);
+    L.total = at;
+    return L;
+}
+
+// Copy `bytes` of a result to the caller's host array: by way of the pinned
+// block while it has room, handed over by sync_and_check.
+rwnmr_status host_out(rwnmr_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    const size_t at = (c->pinned_used + 255) / 256 * 256;
+    if (c->packed_in && at + bytes <= c->pinned.bytes && c->n_results < 10) {   // stage_out needs 6 of the 16
+        RW_HIP(c, hipMemcpyAsync(c->pinned.p + at, src, bytes, hipMemcpyDeviceToHost, c->stream));
+        c->results[c->n_results++] = {dst, c->pinned.p + at, bytes};
+        c->pinned_used = at + bytes;
+        return RWNMR_OK;
+    }
+    RW_HIP(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    return RWNMR_OK;
+}
+
 rwnmr_status stage_in(rwnmr_ctx *c, const rwnmr_walkers *w, WalkerView &v)
 {
     if (w->on_device) {
@@ -332,6 +438,44 @@ rwnmr_status stage_in(rwnmr_ctx *c, const rwnmr_walkers *w, WalkerView &v)
         return RWNMR_OK;
     }
     const uint64_t n = w->n;
+    c->packed_in = false;
+    c->pinned_used = 0;
+    c->n_results = 0;
+    const PackedLayout L = packed_layout(w);
+    if (n && L.total <= kPackedBytes) {
+        // some room for results, in steps of 256 KiB
+        const size_t want = (L.total + (64u << 10) + (256u << 10) - 1) >> 18 << 18;
+        RW_HIP(c, c->packed.reserve(want));
+        // a copy of an earlier call that failed may still read the pinned buffer
+        if (c->staging_open)
+            RW_HIP(c, hipStreamSynchronize(c->stream));
+        if (c->pinned.reserve(want)) {
+            char *h = c->pinned.p, *d = c->packed.as<char>();
+            memcpy(h + L.x, w->x, n * 4);
+            memcpy(h + L.y, w->y, n * 4);
+            memcpy(h + L.z, w->z, n * 4);
+            memcpy(h + L.seed, w->seed, n * 8);
+            if (w->energy)
+                memcpy(h + L.energy, w->energy, n * 8);
+            if (w->hits)
+                memcpy(h + L.hits, w->hits, n * 4);
+            if (w->penalty)
+                memcpy(h + L.penalty, w->penalty, n * 8);
+            c->staging_open = true;
+            RW_HIP(c, hipMemcpyAsync(d, h, L.total, hipMemcpyHostToDevice, c->stream));
+            v.x = (int32_t *)(d + L.x);
+            v.y = (int32_t *)(d + L.y);
+            v.z = (int32_t *)(d + L.z);
+            v.seed = (uint64_t *)(d + L.seed);
+            v.energy = w->energy ? (double *)(d + L.energy) : nullptr;
+            v.hits = w->hits ? (uint32_t *)(d + L.hits) : nullptr;
+            v.penalty = w->penalty ? (const double *)(d + L.penalty) : nullptr;
+            c->packed_in = true;
+            c->packed_at = L;
+            c->pinned_used = L.total;
+            return RWNMR_OK;
+        }
+    }
     RW_HIP(c, c->x.reserve(n * 4 + 4));
     RW_HIP(c, c->y.reserve(n * 4 + 4));
     RW_HIP(c, c->z.reserve(n * 4 + 4));
@@ -370,6 +514,21 @@ rwnmr_status stage_out(rwnmr_ctx *c, rwnmr_walkers *w, const WalkerView &v)
     if (w->on_device)
         return RWNMR_OK;
     const uint64_t n = w->n;
+    if (c->packed_in) {
+        const PackedLayout &L = c->packed_at;
+        const char *d = c->packed.as<char>();
+        char *h = c->pinned.p;
+        RW_HIP(c, hipMemcpyAsync(h, d, L.results, hipMemcpyDeviceToHost, c->stream));
+        c->results[c->n_results++] = {w->x, h + L.x, n * 4};
+        c->results[c->n_results++] = {w->y, h + L.y, n * 4};
+        c->results[c->n_results++] = {w->z, h + L.z, n * 4};
+        c->results[c->n_results++] = {w->seed, h + L.seed, n * 8};
+        if (w->energy)
+            c->results[c->n_results++] = {w->energy, h + L.energy, n * 8};
+        if (w->hits)
+            c->results[c->n_results++] = {w->hits, h + L.hits, n * 4};
+        return RWNMR_OK;
+    }
     RW_HIP(c, hipMemcpyAsync(w->x, v.x, n * 4, hipMemcpyDeviceToHost, c->stream));
     RW_HIP(c, hipMemcpyAsync(w->y, v.y, n * 4, hipMemcpyDeviceToHost, c->stream));
     RW_HIP(c, hipMemcpyAsync(w->z, v.z, n * 4, hipMemcpyDeviceToHost, c->stream));
@@ -963,7 +1122,11 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
             // the previous launch's last echo with identical bits)
             RW_HIP(c, rwnmr::launch_reduce_rows(a.partials, (uint64_t)ne + 1, blocks, sums + done, c->stream));
         }
-        if (jac)
+        if (jac && ne == echoes)
+            // one launch: the labels' rows follow each other on both sides
+            RW_HIP(c, rwnmr::launch_reduce_rows(a.jac_partials, (uint64_t)img->n_labels * ((uint64_t)ne + 1), blocks,
+                                                jrows, c->stream));
+        else if (jac)
             for (int l = 0; l < img->n_labels; ++l)
                 RW_HIP(c, rwnmr::launch_reduce_rows(a.jac_partials + (uint64_t)l * (ne + 1) * blocks, (uint64_t)ne + 1,
                                                     blocks, jrows + (uint64_t)l * (echoes + 1) + done, c->stream));
@@ -972,18 +1135,15 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
     }
     if (!w->on_device) {
         if (echo_sums)
-            RW_HIP(c, hipMemcpyAsync(echo_sums, sums, sizeof(double) * ((size_t)echoes + 1), hipMemcpyDeviceToHost,
-                                     c->stream));
+            RW_ST(host_out(c, echo_sums, sums, sizeof(double) * ((size_t)echoes + 1)));
         if (jac)
-            RW_HIP(c, hipMemcpyAsync(jac, jrows, sizeof(double) * (size_t)img->n_labels * ((size_t)echoes + 1),
-                                     hipMemcpyDeviceToHost, c->stream));
+            RW_ST(host_out(c, jac, jrows, sizeof(double) * (size_t)img->n_labels * ((size_t)echoes + 1)));
         if (emode == 2 && label_hits)
-            RW_HIP(c, hipMemcpyAsync(label_hits, a.label_hits, sizeof(uint32_t) * (size_t)img->n_labels * w->n,
-                                     hipMemcpyDeviceToHost, c->stream));
+            RW_ST(host_out(c, label_hits, a.label_hits, sizeof(uint32_t) * (size_t)img->n_labels * w->n));
         if (emode == 3 && fr->p_alive)
-            RW_HIP(c, hipMemcpyAsync(fr->p_alive, a.p_alive, 8 * w->n, hipMemcpyDeviceToHost, c->stream));
+            RW_ST(host_out(c, fr->p_alive, a.p_alive, 8 * w->n));
         if (emode == 3 && fr->phase)
-            RW_HIP(c, hipMemcpyAsync(fr->phase, a.phase, 8 * w->n, hipMemcpyDeviceToHost, c->stream));
+            RW_ST(host_out(c, fr->phase, a.phase, 8 * w->n));
         if ((s = stage_out(c, w, v)) != RWNMR_OK)
             return s;
         return sync_and_check(c);
@@ -1067,6 +1227,8 @@ void rwnmr_ctx_destroy(rwnmr_ctx *c)
         c->sortA[i].release();
         c->sortB[i].release();
     }
+    c->packed.release();
+    c->pinned.release();
     if (c->host_flag)
         (void)hipHostFree(c->host_flag);
     timing_collect(c);
@@ -1977,7 +2139,7 @@ rwnmr_status rwnmr_cpmg_run_label_sets(rwnmr_ctx *c, const rwnmr_image *img, rwn
         }
     }
     if (!w->on_device) {
-        RW_HIP(c, hipMemcpyAsync(echo_sums, sums, 8 * rows * n_sets, hipMemcpyDeviceToHost, c->stream));
+        RW_ST(host_out(c, echo_sums, sums, 8 * rows * n_sets));
         if ((s = stage_out(c, w, v)) != RWNMR_OK)
             return s;
         return sync_and_check(c);
@@ -2151,10 +2313,10 @@ rwnmr_status pfgse_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w
     }
     if (!w->on_device) {
         if (n_samples)
-            RW_HIP(c, hipMemcpyAsync(M_samples, Ms_dev, 8ull * mrows * n_samples, hipMemcpyDeviceToHost, c->stream));
-        RW_HIP(c, hipMemcpyAsync(M, Mdev, 8ull * mrows, hipMemcpyDeviceToHost, c->stream));
+            RW_ST(host_out(c, M_samples, Ms_dev, 8ull * mrows * n_samples));
+        RW_ST(host_out(c, M, Mdev, 8ull * mrows));
         if (msd)
-            RW_HIP(c, hipMemcpyAsync(msd, msd_dev, 24ull * n_delta, hipMemcpyDeviceToHost, c->stream));
+            RW_ST(host_out(c, msd, msd_dev, 24ull * n_delta));
         if ((s = stage_out(c, w, v)) != RWNMR_OK)
             return s;
         return sync_and_check(c);
