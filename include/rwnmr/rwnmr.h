@@ -63,7 +63,9 @@ rwnmr_status rwnmr_ctx_synchronize(rwnmr_ctx *ctx);
 /* The context's hipStream_t, as an opaque pointer (for event timing). */
 void *rwnmr_ctx_stream(rwnmr_ctx *ctx);
 /* Launch shape for walk kernels: threads per block (64..1024, multiple of
- * 64) and walkers per lane (1, 2 or 4).  0 selects the built-in default. */
+ * 64) and walkers per lane (1, 2 or 4).  0 selects the built-in default: 256 x 1,
+ * 64 x 1 for CPMG / map runs of up to 49,152 walkers, 1024 x 1 for sorted mirror
+ * runs of 524,288 and more. */
 rwnmr_status rwnmr_ctx_set_launch(rwnmr_ctx *ctx, uint32_t threads_per_block, uint32_t walkers_per_lane);
 rwnmr_status rwnmr_ctx_get_launch(const rwnmr_ctx *ctx, uint32_t *threads_per_block, uint32_t *walkers_per_lane);
 /* HIP-event timing of every walk / PFGSE kernel launched on the context
@@ -82,9 +84,11 @@ rwnmr_status rwnmr_ctx_set_image_layout(rwnmr_ctx *ctx, int32_t sx, int32_t sy, 
  * resort_every echoes and tiles are striped so each XCD walks one compact
  * region of the image (its L2 holds that region).  Walker results are
  * identical with it on or off; echo sums differ only in summation order.
- * Default on, every 1000 echoes, from 65,536 walkers. */
+ * Until this is called: every 1000 echoes, from 65,536 walkers, runs of less than
+ * about 2 ms of walk left unsorted.  Internal-field runs (on fields of more than
+ * 4 MiB and 256 steps, until this is called) take the walkers in the same order. */
 rwnmr_status rwnmr_ctx_set_locality(rwnmr_ctx *ctx, int32_t enable, uint32_t resort_every, uint64_t min_walkers);
-/* Periodic and mirror CPMG / map walks (shift 0, uniform or per-walker
+/* Periodic and mirror CPMG / map walks (uniform or per-walker
  * delta) on an unfolded copy of the image: the mirror tiling of period 2d
  * (or the periodic one of period d) stored once with Z-order voxel
  * addresses, so a step needs no fold (replaces the per-step fold of
@@ -93,18 +97,20 @@ rwnmr_status rwnmr_ctx_set_locality(rwnmr_ctx *ctx, int32_t enable, uint32_t res
  * 2^32 voxels use the folded kernels.  mode 0: folded kernels; 1: unfolded;
  * 2: unfolded, each walker also keeping the 16-byte chunk (8 x 4 x 4
  * voxels) of its last lookup in registers so most steps read no memory;
- * 3 (default) and 4: the chunk tested by one shift and the next direction
+ * 3 and 4: the chunk tested by one shift and the next direction
  * drawn a step ahead, through the 4 KiB byte-key table (3) or the 64 KiB
  * wide direction table (4).  Modes 3 and 4 also run noflux walks (image
  * sides >= 2) on the periodic unfolded image, and start mirror CPMG / map
  * walkers at their folded positions with reflection flags (mirrored
- * direction tables, byte-key form).  5: as 3 for every walk except CPMG with
- * one walker per lane, which loads the chunks of both possible next
+ * direction tables, byte-key form).  5: as 3 for every walk except CPMG and
+ * map with one walker per lane, which load the chunks of both possible next
  * candidates a step ahead (two loads per walker-step) and draws directions
- * two steps ahead: for latency-bound runs of few walkers.  6: as 3, with
- * mirror walks keeping an 8-byte chunk (4 x 4 x 4 voxels: 3 VALU per step
- * fewer, a quarter more chunk loads); other walks run as 3.  Results are
- * identical in every mode. */
+ * three steps ahead: for latency-bound runs of few walkers.  6: as 3, with
+ * an 8-byte chunk (4 x 4 x 4 voxels: 3 VALU per step fewer, a quarter more
+ * chunk loads) in walks of one walker per lane and mirror walks.  Until this
+ * or set_launch is called, CPMG and map runs of up to 65,536 walkers take 5,
+ * and larger ones 6 or 3 by size.  Modes 3 and up also walk divided images
+ * (shift > 0).  Walkers are identical in every mode, echo sums to rounding. */
 rwnmr_status rwnmr_ctx_set_unfolded(rwnmr_ctx *ctx, int32_t mode);
 
 /* Upload a packed image in the reference bitBlock layout: block index

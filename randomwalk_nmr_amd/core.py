@@ -74,7 +74,8 @@ class Context:
         check(load().rwnmr_ctx_set_image_layout(self.handle, sx, sy, sz), self.handle)
 
     def set_locality(self, enable: bool = True, resort_every: int = 1000, min_walkers: int = 65536):
-        """Morton ordering of walkers + XCD-striped tiles for large runs."""
+        """Morton ordering of walkers + XCD-striped tiles for large runs.
+        Until this is called, runs too short to gain by it stay unsorted."""
         check(load().rwnmr_ctx_set_locality(self.handle, int(enable), int(resort_every), int(min_walkers)),
               self.handle)
 
@@ -83,12 +84,12 @@ class Context:
         of sides >= 2, on the periodic unfolded image): 0 folded kernels, 1 unfolded image (no
         per-step fold), 2 unfolded + per-walker 16-byte chunk cache, 3 and 4
         the chunk tested by one shift and the next direction drawn a step
-        ahead, through the 4 KiB byte-key table (3, default) or the 64 KiB
-        wide direction table (4); 5 as 3, with CPMG of one walker per lane
+        ahead, through the 4 KiB byte-key table (3) or the 64 KiB
+        wide direction table (4); 5 as 3, with CPMG and map walks of one walker per lane
         loading both possible next chunks a step ahead (latency-bound runs
-        of few walkers); 6 as 3, with mirror walks keeping an 8-byte (4 x 4
-        x 4 voxel) chunk (3 VALU per step fewer, a quarter more chunk
-        loads)."""
+        of few walkers); 6 as 3, with an 8-byte (4 x 4 x 4 voxel) chunk
+        (3 VALU per step fewer, a quarter more chunk loads).  Until this or
+        set_launch is called the run's size chooses 5, 6 or 3."""
         check(load().rwnmr_ctx_set_unfolded(self.handle, int(mode)), self.handle)
 
     def set_timing(self, enable: bool = True):

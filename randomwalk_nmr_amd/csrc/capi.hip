@@ -1772,7 +1772,11 @@ rwnmr_status rwnmr_cpmg_run_noalloc(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_
     a.n_labels = img->n_labels;
     // an unfolded image is used only when an earlier call built it
     attach_zimage(c, img, bc, 1, a, true, true, false);
-    const LaunchShape shape = plan_run(c, a, 1, false);
+    LaunchShape shape = plan_run(c, a, 1, false);
+    // 64-thread blocks have more echo partials: not where these would split the run
+    if (shape.threads < c->shape.threads &&
+        ((uint64_t)echoes + 1) * rwnmr::walk_grid_blocks(w->n, shape, (int)shift) > part_doubles)
+        shape = c->shape;
     const uint32_t blocks = rwnmr::walk_grid_blocks(w->n, shape, (int)shift);
     // echoes per launch: rows 0..chunk of [echo][block] partials must fit the scratch
     uint64_t chunk = echoes ? echoes : 1;
@@ -1866,7 +1870,11 @@ rwnmr_status rwnmr_cpmg_graph_create(rwnmr_ctx *c, const rwnmr_image *img, rwnmr
     WalkArgs a = base_args(img, v, w, 0, c->flag.as<uint32_t>());
     a.n_labels = img->n_labels;
     attach_zimage(c, img, bc, 1, a, true, true, true);
-    const LaunchShape shape = plan_run(c, a, 1, false);
+    LaunchShape shape = plan_run(c, a, 1, false);
+    // 64-thread blocks have more echo partials: not where these would split the run
+    if (shape.threads < c->shape.threads &&
+        ((uint64_t)echoes + 1) * rwnmr::walk_grid_blocks(n, shape, 0) > kMaxPartialBytes / 8)
+        shape = c->shape;
     const uint32_t blocks = rwnmr::walk_grid_blocks(n, shape, 0);
     uint64_t chunk = echoes ? echoes : 1;
     if (echo_sums && blocks)

@@ -133,3 +133,36 @@ def test_division_beyond_32_bit_addresses_takes_the_folded_walk():
     o = O.walk(O.bitblock_pack(solid), dims, x, y, z, seeds, echoes=5, steps_per_echo=50, bc="mirror", shift=8,
                penalty=pen)
     _same(g, o)
+
+
+def test_noalloc_run_that_narrow_blocks_would_split():
+    """40,000 walkers and 4,000 echoes fit the static scratch with 256-thread
+    blocks only; without an energy array the run has to stay one launch."""
+    import ctypes as ct
+
+    import torch
+
+    from randomwalk_nmr_amd._lib import load
+    from randomwalk_nmr_amd.core import _walker_struct, bc_code
+
+    print("[test] noalloc, one launch", flush=True)
+    n, echoes = 40_000, 4000
+    solid, seeds, x, y, z, _ = _inputs((32, 32, 32), n, 8)
+    L = load()
+    out = []
+    with R.Context(0) as ctx:
+        img = R.Image.from_solid(ctx, solid)
+        for fn in (L.rwnmr_cpmg_run, L.rwnmr_cpmg_run_noalloc):
+            t = [torch.from_numpy(v.copy()).to("cuda") for v in (x, y, z, seeds.view(np.int64))]
+            sums = torch.zeros(echoes + 1, dtype=torch.float64, device="cuda")
+            w = _walker_struct(*t, None, None, None, 0.999, n, 1)
+            torch.cuda.synchronize()
+            code = fn(ctx.handle, img.handle, ct.byref(w), echoes, 1, bc_code("mirror"), 0,
+                      ct.c_void_p(sums.data_ptr()))
+            assert code == 0, L.rwnmr_last_error(ctx.handle)
+            ctx.synchronize()
+            out.append([v.cpu().numpy() for v in t] + [sums.cpu().numpy()])
+        img.close()
+    for a, b in zip(out[0][:4], out[1][:4]):
+        assert np.array_equal(a, b)
+    assert np.all(np.abs(out[0][4] - out[1][4]) <= RTOL * out[1][4])
