@@ -847,8 +847,6 @@ rwnmr_status walk_local(rwnmr_ctx *c, const rwnmr_image *img, const WalkArgs &a,
                         uint32_t steps_per_echo, double *sums, uint64_t max_chunk, const LaunchShape &ls)
 {
     const uint64_t n = a.n;
-    if (n > 0xFFFFFFFFull)
-        return fail(c, RWNMR_ERR_INVALID, "locality ordering supports up to 2^32 walkers");
     // a's tiles (balanced tiles when walk_columns set them)
     const uint64_t per_tile = a.tile_walkers ? (uint64_t)a.tile_walkers : (uint64_t)ls.threads * ls.k;
     const uint32_t tiles = (uint32_t)((n + per_tile - 1) / per_tile);
@@ -1039,8 +1037,11 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
     attach_zimage(c, img, bc, emode, a, true, true);
     if (jac && (!a.zwords || !a.zlabels))
         return fail(c, RWNMR_ERR_INVALID, "Jacobian forward: needs the unfolded labelled image");
-    const bool local = emode < 2 && shift == 0 && c->locality && w->n >= c->locality_min_walkers &&
-                       (!c->locality_auto || sorts_pay(w->n, (uint64_t)echoes * steps_per_echo));
+    const bool sorted = emode < 2 && shift == 0 && c->locality && w->n >= c->locality_min_walkers &&
+                        (!c->locality_auto || sorts_pay(w->n, (uint64_t)echoes * steps_per_echo));
+    if (sorted && w->n > 0xFFFFFFFFull)
+        return fail(c, RWNMR_ERR_INVALID, "locality ordering supports up to 2^32 walkers");
+    const bool local = sorted && rwnmr::position_sort_takes(w->n);
     // the Jacobian forward holds one walker per lane
     const LaunchShape shape = jac ? LaunchShape{c->shape.threads, 1u} : plan_run(c, a, emode, local);
     // tiles, one echo-partial column each (balanced tiles where they apply)
@@ -1099,7 +1100,8 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
         a.n_tiles = blocks;
     }
     // field walks in position order
-    const bool ordered = emode == 3 && c->locality && w->n >= c->locality_min_walkers && w->n <= 0xFFFFFFFFull &&
+    const bool ordered = emode == 3 && c->locality && w->n >= c->locality_min_walkers &&
+                         rwnmr::position_sort_takes(w->n) &&
                          (!c->locality_auto || field_order_pays(img, (uint64_t)echoes * steps_per_echo));
     if (ordered)
         chunk = std::min<uint64_t>(chunk, std::max<uint32_t>(1u, c->resort_every));

@@ -100,6 +100,8 @@ hipError_t launch_morton_keys(int bc, const int32_t *x, const int32_t *y, const 
 
 hipError_t sort_pairs_temp_bytes(uint64_t n, int end_bit, size_t *bytes)
 {
+    if (!position_sort_takes(n))
+        return hipErrorInvalidValue;
     return hipcub::DeviceRadixSort::SortPairs(nullptr, *bytes, (const uint32_t *)nullptr, (uint32_t *)nullptr,
                                               (const uint32_t *)nullptr, (uint32_t *)nullptr, (int)n, 0, end_bit);
 }
@@ -107,6 +109,8 @@ hipError_t sort_pairs_temp_bytes(uint64_t n, int end_bit, size_t *bytes)
 hipError_t sort_pairs(void *temp, size_t bytes, const uint32_t *keys_in, uint32_t *keys_out, const uint32_t *vals_in,
                       uint32_t *vals_out, uint64_t n, int end_bit, hipStream_t st)
 {
+    if (!position_sort_takes(n))
+        return hipErrorInvalidValue;
     return hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys_in, keys_out, vals_in, vals_out, (int)n, 0, end_bit,
                                               st);
 }

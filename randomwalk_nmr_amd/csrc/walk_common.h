@@ -161,6 +161,10 @@ RW_HD uint32_t morton3(uint32_t bx, uint32_t by, uint32_t bz)
     return spread3(bx) | (spread3(by) << 1) | (spread3(bz) << 2);
 }
 
+// Whether the position sort takes n walkers: its indices are 32 bits and the
+// radix sort counts its items in an int.  More walkers walk in their own order.
+RW_HD bool position_sort_takes(uint64_t n) { return n <= 0x7FFFFFFFull; }
+
 // ------------------------------------------------------------------------
 // Unfolded image with dilated voxel addresses (periodic and mirror walks).
 //

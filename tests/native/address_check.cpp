@@ -3,6 +3,7 @@
 // a noflux move turns around exactly where a walker in a face voxel would step
 // outwards, and a sub-voxel address shifted by 3 bits per division is the
 // undivided image's address of the walker's voxel, mirror reflection included.
+// Also: the walker counts whose position sort fits its int item count.
 #include <cstdio>
 #include <cstdlib>
 
@@ -60,6 +61,9 @@ int main()
                     EXPECT(fold_periodic(g, (int)n[a]) >> shift == fold_periodic(g >> shift, (int)d[a]), "periodic\n");
                 }
         }
+    const uint64_t counts[] = {0ull, 1ull, 0x7FFFFFFFull, 0x80000000ull, 0xFFFFFFFFull, 0x100000000ull, 0x100000001ull};
+    for (uint64_t n : counts)
+        EXPECT(position_sort_takes(n) == (n < (1ull << 31)), "sort of %llu\n", (unsigned long long)n);
     std::printf("%ld checks, %ld failures\n", checks, fails);
     return fails ? 1 : 0;
 }
