@@ -89,6 +89,8 @@ __global__ __launch_bounds__(256) void scatter_walkers_kernel(SortedState out, S
 hipError_t launch_morton_keys(int bc, const int32_t *x, const int32_t *y, const int32_t *z, uint64_t n, int W, int H,
                               int D, uint32_t *keys, uint32_t *iota, hipStream_t st)
 {
+    if (n == 0)
+        return hipSuccess;
     const uint32_t grid = (uint32_t)((n + 255) / 256);
     switch (bc) {
     case kNoflux: hipLaunchKernelGGL(morton_keys_kernel<kNoflux>, dim3(grid), dim3(256), 0, st, x, y, z, n, W, H, D, keys, iota); break;
@@ -102,6 +104,9 @@ hipError_t sort_pairs_temp_bytes(uint64_t n, int end_bit, size_t *bytes)
 {
     if (!position_sort_takes(n))
         return hipErrorInvalidValue;
+    *bytes = 0;
+    if (n == 0)
+        return hipSuccess;
     return hipcub::DeviceRadixSort::SortPairs(nullptr, *bytes, (const uint32_t *)nullptr, (uint32_t *)nullptr,
                                               (const uint32_t *)nullptr, (uint32_t *)nullptr, (int)n, 0, end_bit);
 }
@@ -111,6 +116,8 @@ hipError_t sort_pairs(void *temp, size_t bytes, const uint32_t *keys_in, uint32_
 {
     if (!position_sort_takes(n))
         return hipErrorInvalidValue;
+    if (n == 0)
+        return hipSuccess;
     return hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys_in, keys_out, vals_in, vals_out, (int)n, 0, end_bit,
                                               st);
 }
@@ -118,6 +125,8 @@ hipError_t sort_pairs(void *temp, size_t bytes, const uint32_t *keys_in, uint32_
 hipError_t launch_gather_walkers(const SortedState &dst, const SortedState &src, const uint32_t *perm,
                                  const uint32_t *orig_src, const double *penalty, uint64_t n, hipStream_t st)
 {
+    if (n == 0)
+        return hipSuccess;
     hipLaunchKernelGGL(gather_walkers_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, dst, src, perm,
                        orig_src, penalty, n);
     return hipGetLastError();
@@ -125,6 +134,8 @@ hipError_t launch_gather_walkers(const SortedState &dst, const SortedState &src,
 
 hipError_t launch_scatter_walkers(const SortedState &out, const SortedState &s, uint64_t n, hipStream_t st)
 {
+    if (n == 0)
+        return hipSuccess;
     hipLaunchKernelGGL(scatter_walkers_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, out, s, n);
     return hipGetLastError();
 }

@@ -38,3 +38,22 @@ def test_field_walk_in_position_order(bc, n, echoes):
         for k in ("x", "y", "z", "seed", "hits", "p_alive", "phase", "energy"):
             assert np.array_equal(np.asarray(out[0][k]).view(np.uint8), np.asarray(o[k]).view(np.uint8)), k
         assert np.all(np.abs(out[0]["echo_sums"] - o["echo_sums"]) <= 1e-12 * n)
+
+
+@pytest.mark.parametrize("bc", ["noflux", "periodic", "mirror"])
+def test_no_walkers_in_position_order(bc):
+    """A context that orders every run takes one without walkers: echo sums of 0."""
+    print(f"[test] no walkers, ordered, bc={bc}", flush=True)
+    rng = np.random.default_rng(1)
+    solid = (rng.random((24, 32, 40)) < 0.3).astype(np.uint8)
+    none = np.zeros(0, np.int32)
+    w = (none, none, none, np.zeros(0, np.uint64))
+    with R.Context(0) as ctx:
+        ctx.set_locality(True, 10, 0)
+        img = R.Image.from_solid(ctx, solid)
+        f = R.cpmg_field_run(ctx, img, *w, echoes=25, steps_per_echo=4, field=rng.normal(size=solid.shape),
+                             gyromagnetic_ratio=42.576, time_interval_ms=0.01, bc=bc)
+        g = R.cpmg_run(ctx, img, *w, echoes=25, steps_per_echo=4, bc=bc)
+        img.close()
+    for o in (f, g):
+        assert o["echo_sums"].shape == (26,) and not np.any(o["echo_sums"])
