@@ -797,10 +797,13 @@ __device__ __forceinline__ void zwalk_tile(const WalkArgs &a, uint64_t tile, dou
                 return;
             }
             if (CACHE >= 64) {
-                // wall is a mask here: no branch but the label's load
+                // wall is a mask here: no branch but the label's load.  A packed
+                // displacement is selected like the address: the sum runs
+                // beside the wall test (map, 160x130x95, 300k walkers: 295 ns
+                // per step against 313 with the addend masked after it)
                 A[k] = zsel(wall, A[k], C[k]);
                 if (DISP)
-                    P[k] += (int32_t)((uint32_t)DP[k] & ~wall);
+                    P[k] = (int32_t)zsel(wall, (uint32_t)P[k], (uint32_t)(P[k] + DP[k]));
                 if (HITS)
                     Hc[k] -= wall;
                 if (EMODE == 1)
