@@ -10,7 +10,7 @@ template hipError_t launch_z_mode<2>(const WalkArgs &, const LaunchShape &, uint
 // Label-set CPMG: 8 sets of label deltas evaluated on one trajectory (one
 // walker per lane; zwalk_tile with NS = 8).  Unused sets (a.n_label_sets <
 // 8) carry deltas of 1.
-template <bool WRAPFIX, bool NOFLUX, bool MFLAGS, bool ADISP>
+template <bool WRAPFIX, bool NOFLUX, bool MFLAGS>
 __global__ __launch_bounds__(1024) void zwalk_sets_kernel(const WalkArgs a)
 {
     extern __shared__ double lds8[];   // kEchoChunk x 8 sets x waves of the block
@@ -33,7 +33,7 @@ __global__ __launch_bounds__(1024) void zwalk_sets_kernel(const WalkArgs a)
         ldelta[t] = (q < a.n_label_sets && (int)l < a.n_labels) ? a.label_delta[q * (uint32_t)a.n_labels + l] : 1.0;
     }
     __syncthreads();
-    zwalk_tile<2, 1, WRAPFIX, 128, 2, NOFLUX, MFLAGS, 8, false, ADISP>(a, tile, a.partials ? a.partials + tile : nullptr,
+    zwalk_tile<2, 1, WRAPFIX, 128, 2, NOFLUX, MFLAGS, 8>(a, tile, a.partials ? a.partials + tile : nullptr,
                                                          a.partial_stride, nullptr, tab, fix, ldelta, keys, nullptr,
                                                          lds8);
 }
@@ -42,7 +42,7 @@ __global__ __launch_bounds__(1024) void zwalk_sets_kernel(const WalkArgs a)
 // per lane, per-label hit counts in LDS) that also sums h_l E per label and
 // echo (zwalk_tile JAC).  Dynamic LDS: the 8-label echo staging (kEchoChunk
 // x 8 x waves doubles), then the hit-count rows (blockDim x kLhStride).
-template <bool WRAPFIX, bool NOFLUX, bool MFLAGS, bool ADISP>
+template <bool WRAPFIX, bool NOFLUX, bool MFLAGS>
 __global__ __launch_bounds__(1024) void zwalk_jac_kernel(const WalkArgs a)
 {
     extern __shared__ double zjdyn[];
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(1024) void zwalk_jac_kernel(const WalkArgs a)
     if (threadIdx.x < kMaxLabels)
         ldelta[threadIdx.x] = (int)threadIdx.x < a.n_labels ? a.label_delta[threadIdx.x] : 1.0;
     __syncthreads();
-    zwalk_tile<2, 1, WRAPFIX, 128, 2, NOFLUX, MFLAGS, 1, true, ADISP>(a, tile, a.partials ? a.partials + tile : nullptr,
+    zwalk_tile<2, 1, WRAPFIX, 128, 2, NOFLUX, MFLAGS, 1, true>(a, tile, a.partials ? a.partials + tile : nullptr,
                                                                a.partial_stride, lds, tab, fix, ldelta, keys, zlh,
                                                                lds8);
 }
@@ -85,24 +85,17 @@ hipError_t launch_zwalk_sets(const WalkArgs &a, uint32_t threads, hipStream_t st
     // the per-set echo staging, sized for this block's waves
     const size_t lds8_bytes = (size_t)kEchoChunk * 8 * (threads / kWave) * sizeof(double);
     const dim3 g(blocks), b(threads);
-    const bool disp = zaddress_displacement_ok(a.zl);
-#define RW_SETS(WF, MF)                                                                                  \
-    do {                                                                                                 \
-        if (disp)                                                                                        \
-            hipLaunchKernelGGL((zwalk_sets_kernel<WF, false, MF, true>), g, b, lds8_bytes, st, a);       \
-        else                                                                                             \
-            hipLaunchKernelGGL((zwalk_sets_kernel<WF, false, MF, false>), g, b, lds8_bytes, st, a);      \
-    } while (0)
+#define RW_SETS(WF, NF, MF) hipLaunchKernelGGL((zwalk_sets_kernel<WF, NF, MF>), g, b, lds8_bytes, st, a)
     if (a.znoflux)
-        hipLaunchKernelGGL((zwalk_sets_kernel<false, true, false, false>), g, b, lds8_bytes, st, a);
+        RW_SETS(false, true, false);
     else if (a.zmflags && a.zl.wrapfix)
-        RW_SETS(true, true);
+        RW_SETS(true, false, true);
     else if (a.zmflags)
-        RW_SETS(false, true);
+        RW_SETS(false, false, true);
     else if (a.zl.wrapfix)
-        RW_SETS(true, false);
+        RW_SETS(true, false, false);
     else
-        RW_SETS(false, false);
+        RW_SETS(false, false, false);
 #undef RW_SETS
     return hipGetLastError();
 }
@@ -121,24 +114,17 @@ hipError_t launch_zwalk_jac(const WalkArgs &a, uint32_t threads, hipStream_t st)
     const size_t dyn = (size_t)kEchoChunk * 8 * (threads / kWave) * sizeof(double) +
                        (size_t)kLhStride * threads * sizeof(uint32_t);
     const dim3 g(blocks), b(threads);
-    const bool disp = zaddress_displacement_ok(a.zl);
-#define RW_JAC(WF, MF)                                                                            \
-    do {                                                                                          \
-        if (disp)                                                                                 \
-            hipLaunchKernelGGL((zwalk_jac_kernel<WF, false, MF, true>), g, b, dyn, st, a);        \
-        else                                                                                      \
-            hipLaunchKernelGGL((zwalk_jac_kernel<WF, false, MF, false>), g, b, dyn, st, a);       \
-    } while (0)
+#define RW_JAC(WF, NF, MF) hipLaunchKernelGGL((zwalk_jac_kernel<WF, NF, MF>), g, b, dyn, st, a)
     if (a.znoflux)
-        hipLaunchKernelGGL((zwalk_jac_kernel<false, true, false, false>), g, b, dyn, st, a);
+        RW_JAC(false, true, false);
     else if (a.zmflags && a.zl.wrapfix)
-        RW_JAC(true, true);
+        RW_JAC(true, false, true);
     else if (a.zmflags)
-        RW_JAC(false, true);
+        RW_JAC(false, false, true);
     else if (a.zl.wrapfix)
-        RW_JAC(true, false);
+        RW_JAC(true, false, false);
     else
-        RW_JAC(false, false);
+        RW_JAC(false, false, false);
 #undef RW_JAC
     return hipGetLastError();
 }

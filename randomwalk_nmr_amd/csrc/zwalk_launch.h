@@ -68,16 +68,17 @@ static hipError_t launch_z(const WalkArgs &a, const LaunchShape &ls, uint32_t bl
 {
     // EMODE 2 with one walker per lane keeps the per-label hit counts in LDS
     const size_t lh_bytes = EMODE == 2 ? (size_t)kLhStride * ls.threads * sizeof(uint32_t) : 0;
-    // one walker per lane on images of periods of 128 and more: unbounded
-    // moves from address displacements; hits counted only when asked for
-    if constexpr (CACHE >= 64 && TAB >= 2 && !NOFLUX) {
+    // CPMG and map walks of one walker per lane on images of periods of 128 and
+    // more: unbounded moves from address displacements; hits counted only when
+    // asked for
+    if constexpr (EMODE < 2 && CACHE >= 64 && TAB >= 2 && !NOFLUX) {
         if (ls.k == 1 && zaddress_displacement_ok(a.zl)) {
             if (EMODE == 0 || a.hits)
                 hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, true>), dim3(blocks),
-                                   dim3(ls.threads), lh_bytes, st, a);
+                                   dim3(ls.threads), 0, st, a);
             else
                 hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, true, EMODE == 0>),
-                                   dim3(blocks), dim3(ls.threads), lh_bytes, st, a);
+                                   dim3(blocks), dim3(ls.threads), 0, st, a);
             return hipGetLastError();
         }
     }
@@ -106,8 +107,9 @@ template <int EMODE, bool WRAPFIX, bool NOFLUX, bool MFLAGS>
 static hipError_t launch_z_sub(const WalkArgs &a, const LaunchShape &ls, uint32_t blocks, hipStream_t st)
 {
     const size_t lh_bytes = EMODE == 2 ? (size_t)kLhStride * ls.threads * sizeof(uint32_t) : 0;
-    if (!NOFLUX && zaddress_displacement_ok(a.zl))
-        hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, 64, 2, NOFLUX, MFLAGS, !NOFLUX, true, true>),
+    constexpr bool ADISP = EMODE < 2 && !NOFLUX;
+    if (ADISP && zaddress_displacement_ok(a.zl))
+        hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, 64, 2, NOFLUX, MFLAGS, ADISP, true, true>),
                            dim3(blocks), dim3(ls.threads), lh_bytes, st, a);
     else
         hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, 64, 2, NOFLUX, MFLAGS, false, true, true>), dim3(blocks),
