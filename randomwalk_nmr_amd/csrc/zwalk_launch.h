@@ -70,9 +70,11 @@ static hipError_t launch_z(const WalkArgs &a, const LaunchShape &ls, uint32_t bl
     const size_t lh_bytes = EMODE == 2 ? (size_t)kLhStride * ls.threads * sizeof(uint32_t) : 0;
     // CPMG and map walks of one walker per lane on images of periods of 128 and
     // more: unbounded moves from address displacements; hits counted only when
-    // asked for
+    // asked for.  CPMG outside the flag-keyed tables pairs them with masks,
+    // which more waves per SIMD outrun: up to kZMaskWalkers.
     if constexpr (EMODE < 2 && CACHE >= 64 && TAB >= 2 && !NOFLUX) {
-        if (ls.k == 1 && zaddress_displacement_ok(a.zl)) {
+        const bool few = EMODE == 0 || TAB == 3 || a.n <= kZMaskWalkers;
+        if (few && ls.k == 1 && zaddress_displacement_ok(a.zl)) {
             if (EMODE == 0 || a.hits)
                 hipLaunchKernelGGL((zwalk_kernel<EMODE, 1, WRAPFIX, CACHE, TAB, NOFLUX, MFLAGS, true>), dim3(blocks),
                                    dim3(ls.threads), 0, st, a);
