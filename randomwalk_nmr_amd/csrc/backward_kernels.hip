@@ -170,11 +170,13 @@ __global__ __launch_bounds__(kZBackThreads) void zbackward_kernel(const WalkArgs
         // overlaps the chunk load's
         __builtin_amdgcn_sched_barrier(0);
         settle();
-        const uint32_t wall = zchunk_wall<128>(c, QV);
-        A = zsel(wall, A, c);
-        if (__builtin_expect(wall != 0u, 0)) {
+        // (the label's load branches in any case: a select for the move
+        // beside it made the replay 1% slower)
+        if (__builtin_expect(zchunk_wall<128>(c, QV) != 0u, 0)) {
             lab = zlabel_at(a, c);
             pend = true;
+        } else {
+            A = c;
         }
     };
     const uint32_t e0 = seg * b.every;
