@@ -38,9 +38,9 @@ __host__ __device__ inline bool zaddress_displacement_ok(const ZLayout &zl)
 // CPMG walks with address displacements resolve a wall by masks: no branch,
 // but the energy's product and selects at every step.  With few waves per SIMD
 // (1024 SIMDs x 64 lanes each) waiting is what costs and masks win (96^3,
-// 100k walkers: 227 against 250 ns per step); with many the instructions do,
+// 100k walkers: 234 against 256 ns per step); with many the instructions do,
 // and two short paths with a packed displacement win (128x160x130 periodic:
-// 400k walkers 433 against 448, 1M 973 against 989; 300k 347 against 348 with
+// 400k walkers 433 against 448, 1M 973 against 989; 300k 349 both with
 // the 16-byte chunk, 344 against 336 with the 8-byte one), so the line lies at
 // 5 waves.
 static constexpr uint64_t kZMaskWalkers = 5ull * 1024ull * 64ull;
