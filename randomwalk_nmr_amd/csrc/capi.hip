@@ -757,6 +757,31 @@ rwnmr_status order_by_position(rwnmr_ctx *c, const rwnmr_image *img, WalkArgs &a
     return RWNMR_OK;
 }
 
+// Walkers up to which an unsorted run gains by the 8-byte chunk: scattered
+// lanes share no chunks, so its additional loads queue up in the L2 from a
+// certain number on, the sooner the less of the image the L1s hold.  Time of
+// the 16-byte chunk over the 8-byte one, noflux / periodic / mirror:
+//   map:  64^3    1M    1.10 1.09 1.07
+//         96^3    500k  1.06 1.05 1.01    700k 0.92 0.92 0.89
+//         160x130x95  250k 1.05 1.02 1.00    350k 0.95 0.95 0.92
+//         128^3   200k  1.10 1.05 1.05    250k 1.03 0.95 0.95
+//         256^3   200k  1.05 0.98 1.00    250k 0.92 0.89 0.93
+//   CPMG: 64^3    1M    1.07 1.07 1.06
+//         96^3    500k  1.05 1.06 1.04    700k 1.05 1.01 0.97
+//         160x130x95  400k 1.03 0.99 1.01    500k 1.01 0.98 0.99
+//         160^3   300k  1.05 1.02 1.02    350k 0.99 0.97 0.97
+//         256^3   200k  1.06 1.02 1.05    300k 1.00 0.91 0.94
+uint64_t chunk8_walkers(uint64_t voxels, int emode)
+{
+    if (voxels <= 1ull << 18)
+        return ~0ull;
+    if (voxels <= 1ull << 20)
+        return 500000;
+    if (emode == 0)
+        return voxels < 1ull << 21 ? 250000 : 200000;
+    return voxels < 1ull << 21 ? 400000 : (voxels <= 1ull << 23 ? 300000 : 200000);
+}
+
 // Launch shape of a CPMG, map or per-label run (a as attach_zimage left it)
 // and, where no image form was asked for, the form of a chunk-cache walk.
 // `sorted`: the walkers are kept in position order.
@@ -765,16 +790,14 @@ rwnmr_status order_by_position(rwnmr_ctx *c, const rwnmr_image *img, WalkArgs &a
 //    (128^3, 30k walkers: 152 ns per step against 176 with 256 threads;
 //    65,536 walkers: 178 against 167).
 //  - The 8-byte chunk (form 6) saves 3 instructions per step and costs a
-//    quarter more chunk loads, which pays where these hit the L2: where the
-//    part of the image that is read fits the 4 MiB of one XCD, 3-9% faster up
-//    to 300k walkers and, sorted, at 1M (256^3 mirror, 3 steps per echo: 789
-//    against 855 ns per step), but slower for 1M unsorted ones (1071 against
-//    985) and on a 512^3 mirror image (16 MiB; 1M sorted: 5% slower).
+//    quarter more chunk loads, which pays where these hit the L2: sorted runs
+//    whose part of the image that is read fits the 4 MiB of one XCD (256^3
+//    mirror, 1M walkers, 3 steps per echo: 789 against 855 ns per step; a 512^3
+//    mirror image, 16 MiB: 5% slower), unsorted ones up to chunk8_walkers.
 //  - Sorted mirror walks of a whole round of resident 1024-thread blocks
 //    (512 of them) take the flag-keyed tables of that block size (1M walkers,
 //    12 steps per echo: 746 against 873 ns per step with 256 threads; 300k:
 //    350 against 283).
-constexpr uint64_t kChunk8Unsorted = 400000;
 constexpr uint32_t kChunk8ImageBits = 25;   // log2 of the addresses of 4 MiB
 
 LaunchShape plan_run(const rwnmr_ctx *c, WalkArgs &a, int emode, bool sorted)
@@ -789,7 +812,8 @@ LaunchShape plan_run(const rwnmr_ctx *c, WalkArgs &a, int emode, bool sorted)
     if (c->form_auto && a.zwords && a.zcache == 2 && (ls.k == 1 || a.shift)) {
         // addresses of the base image, of its first octant with reflection flags
         const uint32_t read_bits = a.zl.bits - 3u * (uint32_t)a.shift - (a.zmflags ? 3u : 0u);
-        if (read_bits <= kChunk8ImageBits && (sorted || a.n <= kChunk8Unsorted))
+        const uint64_t voxels = (uint64_t)a.W * (uint64_t)a.H * (uint64_t)a.D;
+        if (read_bits <= kChunk8ImageBits && (sorted || a.n <= chunk8_walkers(voxels, emode)))
             a.zcache = 5;
     }
     return ls;

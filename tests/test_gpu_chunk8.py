@@ -60,3 +60,32 @@ def test_unconfigured_runs_match_named_forms(bc, n, steps):
     for k in ("x", "y", "z", "seed", "hits", "energy"):
         assert np.array_equal(out[0][k], out[1][k]), k
     assert np.all(np.abs(out[0]["echo_sums"] - out[1]["echo_sums"]) <= RTOL * out[1]["echo_sums"])
+
+
+@pytest.mark.parametrize("dims,n", [((64, 64, 64), 262_145), ((96, 96, 96), 500_000), ((96, 96, 96), 500_001),
+                                    ((127, 128, 128), 250_001), ((127, 128, 128), 400_001),
+                                    ((128, 128, 128), 200_001), ((128, 128, 128), 300_001),
+                                    ((128, 160, 130), 327_680), ((128, 160, 130), 327_681)])
+@pytest.mark.parametrize("bc", ["periodic", "mirror"])
+def test_unsorted_lines_match_the_plain_form(dims, n, bc):
+    """Image sizes and walker counts at which an unsorted run changes its chunk,
+    and a CPMG run its way to resolve a wall, against the unfolded walk without
+    a chunk cache: one more flush than the shortest interval, odd step counts."""
+    print(f"[test] unsorted lines bc={bc} dims={dims} n={n}", flush=True)
+    solid, seeds, x, y, z, pen = _inputs(dims, n, 9)
+    out = []
+    for asked in (False, True):
+        with R.Context(0) as ctx:
+            if asked:
+                ctx.set_unfolded(1)
+                ctx.set_launch(256, 1)
+                ctx.set_locality(False)
+            img = R.Image.from_solid(ctx, solid)
+            out.append(R.cpmg_run(ctx, img, x, y, z, seeds, echoes=3, steps_per_echo=43, bc=bc, penalty=pen))
+            m = R.map_run(ctx, img, x, y, z, seeds, steps=129, bc=bc)
+            img.close()
+        for k in ("x", "y", "z", "seed", "hits"):
+            assert np.array_equal(m[k], out[-1][k]), k
+    for k in ("x", "y", "z", "seed", "hits", "energy"):
+        assert np.array_equal(out[0][k], out[1][k]), k
+    assert np.all(np.abs(out[0]["echo_sums"] - out[1]["echo_sums"]) <= RTOL * out[1]["echo_sums"])
