@@ -108,8 +108,8 @@ rwnmr_status rwnmr_ctx_set_locality(rwnmr_ctx *ctx, int32_t enable, uint32_t res
  * three steps ahead: for latency-bound runs of few walkers.  6: as 3, with
  * an 8-byte chunk (4 x 4 x 4 voxels: 3 VALU per step fewer, a quarter more
  * chunk loads) in walks of one walker per lane and mirror walks.  Until this
- * or set_launch is called, CPMG and map runs of up to 65,536 walkers take 5,
- * and larger ones 6 or 3 by size.  Modes 3 and up also walk divided images
+ * or set_launch is called, CPMG runs of up to 65,536 and map runs of up to
+ * 49,152 walkers take 5, and larger ones 6 or 3 by size.  Modes 3 and up also walk divided images
  * (shift > 0).  Walkers are identical in every mode, echo sums to rounding. */
 rwnmr_status rwnmr_ctx_set_unfolded(rwnmr_ctx *ctx, int32_t mode);
 

@@ -650,11 +650,15 @@ const uint8_t *zlabels_for(rwnmr_ctx *c, const rwnmr_image *img, int bc)
 }
 
 // Walker counts up to one wave per SIMD (1024 SIMDs x 64 lanes) take the
-// speculative walk (form 5), with its two loads per step: 139 against 203 ns
-// per step of 10k walkers at 128^3 (mirror), 167 against 197 at 65,536, but
-// 245 against 222 at 100k and 545 against 297 at 200k, where the loads of
-// several waves per SIMD queue up.  The autotuner times it up to here too.
-constexpr uint64_t kSpecMaxWalkers = 1024ull * 64ull;
+// speculative walk (form 5), with its two loads per step: CPMG of 10k walkers
+// at 128^3 (mirror) 139 against 203 ns per step, of 65,536 191 against 196,
+// but 245 against 222 at 100k and 545 against 297 at 200k, where the loads of
+// several waves per SIMD queue up.  A map step waits for less, so there its
+// line lies where the last SIMD of a CU gets a wave: 49,152 walkers 138 against
+// 166, 53,000 171 against 166, 65,536 177 against 166 (64^3 periodic: 126
+// against 141, 159 against 142, 161 against 144).  The autotuner times it up
+// to one wave per SIMD too.
+constexpr uint64_t kSpecMaxWalkers = 1024ull * 64ull, kSpecMaxMapWalkers = 768ull * 64ull;
 
 // Use the unfolded-image kernel for this walk when one applies.  noflux_ok:
 // the caller's kernel also runs noflux walks on the periodic unfolded image
@@ -701,7 +705,8 @@ void attach_zimage(rwnmr_ctx *c, const rwnmr_image *img, int bc, int emode, Walk
         a.zl = z->zl;
         a.zcache = c->unfolded >= 2 ? (uint32_t)(c->unfolded - 1) : 0u;
         // few walkers: the speculative walk, unless a form or a shape was asked for
-        if (c->form_auto && c->shape_auto && emode < 2 && a.n <= kSpecMaxWalkers)
+        if (c->form_auto && c->shape_auto && emode < 2 &&
+            a.n <= (emode == 0 ? kSpecMaxMapWalkers : kSpecMaxWalkers))
             a.zcache = 4;
         a.zlabels = zlab;
         // mirror image of equal power-of-two periods: labels kept for the

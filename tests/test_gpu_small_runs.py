@@ -63,6 +63,20 @@ def test_walker_counts_that_choose_the_form(n):
     assert np.all(np.abs(out[0]["echo_sums"] - out[1]["echo_sums"]) <= RTOL * out[1]["echo_sums"])
 
 
+@pytest.mark.parametrize("n", [49_152, 49_153])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_walker_counts_that_choose_the_form_of_a_map(n, shift):
+    print(f"[test] form choice of a map n={n} shift={shift}", flush=True)
+    dims = (40, 32, 24)
+    solid, seeds, x, y, z, _ = _inputs(dims, n, 9, shift)
+    with R.Context(0) as ctx:
+        img = R.Image.from_solid(ctx, solid)
+        m = R.map_run(ctx, img, x, y, z, seeds, steps=101, bc="mirror", shift=shift)
+        img.close()
+    o = O.walk(O.bitblock_pack(solid), dims, x, y, z, seeds, echoes=1, steps_per_echo=101, bc="mirror", shift=shift)
+    _same(m, o)
+
+
 @pytest.mark.parametrize("threads", [64, 192, 1024])
 def test_speculative_walk_sums_over_several_waves(threads):
     print(f"[test] speculative walk threads={threads}", flush=True)
