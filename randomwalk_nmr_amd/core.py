@@ -88,8 +88,8 @@ class Context:
         wide direction table (4); 5 as 3, with CPMG and map walks of one walker per lane
         loading both possible next chunks a step ahead (latency-bound runs
         of few walkers); 6 as 3, with an 8-byte (4 x 4 x 4 voxel) chunk
-        (3 VALU per step fewer, a quarter more chunk loads).  Until this or
-        set_launch is called the run's size chooses 5, 6 or 3."""
+        (3 VALU per step fewer, a quarter more chunk loads).  Until this is
+        called the run's size chooses 5, 6 or 3."""
         check(load().rwnmr_ctx_set_unfolded(self.handle, int(mode)), self.handle)
 
     def set_timing(self, enable: bool = True):
@@ -118,7 +118,8 @@ class Context:
         return t.value, k.value, ms.value
 
     def get_tuning(self):
-        """(threads_per_block, walkers_per_lane, unfolded_mode, resort_every) now in use
+        """(threads_per_block, walkers_per_lane, unfolded_mode, resort_every): as set, or
+        where they are automatic as the last CPMG or map run took them
         (rwnmr_ctx_get_tuning)."""
         t, k, r = ct.c_uint32(), ct.c_uint32(), ct.c_uint32()
         u = ct.c_int32()

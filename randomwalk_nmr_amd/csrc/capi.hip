@@ -157,6 +157,10 @@ struct rwnmr_ctx {
     LaunchShape shape{256, 1};
     // no shape / no image form was asked for: plan_run and attach_zimage choose by the run
     bool shape_auto = true, form_auto = true;
+    // what the last CPMG or map run on an unfolded image took (threads 0: none
+    // since the context or its settings were made)
+    LaunchShape ran_shape{0, 0};
+    int ran_form = 0;
     // walker staging for host-pointer calls
     DevBuf x, y, z, seed, energy, hits, penalty, x0, y0, z0;
     // per-call small arrays and reductions
@@ -704,8 +708,12 @@ void attach_zimage(rwnmr_ctx *c, const rwnmr_image *img, int bc, int emode, Walk
         a.zwords = z->words;
         a.zl = z->zl;
         a.zcache = c->unfolded >= 2 ? (uint32_t)(c->unfolded - 1) : 0u;
-        // few walkers: the speculative walk, unless a form or a shape was asked for
-        if (c->form_auto && c->shape_auto && emode < 2 &&
+        // few walkers: the speculative walk, unless a form was asked for or a
+        // shape in which it loses to the chunk cache (8k to 65,536 walkers on
+        // 32^3 to 256^3, 256 threads: CPMG 0.75-1.02 of the chunk walk's time,
+        // maps up to 1.15 of it; 64 threads: 0.65-0.9 of it, both)
+        const bool spec_shape = c->shape_auto || (c->shape.k == 1 && c->shape.threads <= (emode == 0 ? 64u : 256u));
+        if (c->form_auto && spec_shape && emode < 2 &&
             a.n <= (emode == 0 ? kSpecMaxMapWalkers : kSpecMaxWalkers))
             a.zcache = 4;
         a.zlabels = zlab;
@@ -805,7 +813,7 @@ uint64_t chunk8_walkers(uint64_t voxels, int emode)
 //    350 against 283).
 constexpr uint32_t kChunk8ImageBits = 25;   // log2 of the addresses of 4 MiB
 
-LaunchShape plan_run(const rwnmr_ctx *c, WalkArgs &a, int emode, bool sorted)
+LaunchShape plan_run(rwnmr_ctx *c, WalkArgs &a, int emode, bool sorted)
 {
     LaunchShape ls = c->shape;
     if (c->shape_auto && a.zwords && emode < 2) {
@@ -821,8 +829,18 @@ LaunchShape plan_run(const rwnmr_ctx *c, WalkArgs &a, int emode, bool sorted)
         if (read_bits <= kChunk8ImageBits && (sorted || a.n <= chunk8_walkers(voxels, emode)))
             a.zcache = 5;
     }
+    if (a.zwords && emode < 2) {
+        c->ran_shape = ls;
+        c->ran_form = (int)a.zcache + 1;
+    }
     return ls;
 }
+
+// The launch shape and image form that a CPMG run like the last one takes: the
+// settings, or where these are automatic what that run took.
+LaunchShape shape_in_use(const rwnmr_ctx *c) { return c->shape_auto && c->ran_shape.threads ? c->ran_shape : c->shape; }
+
+int form_in_use(const rwnmr_ctx *c) { return c->form_auto && c->ran_shape.threads ? c->ran_form : c->unfolded; }
 
 hipError_t launch_any_walk(const WalkArgs &a, int bc, int emode, const LaunchShape &ls, hipStream_t st)
 {
@@ -1300,6 +1318,7 @@ rwnmr_status rwnmr_ctx_set_unfolded(rwnmr_ctx *c, int32_t enable)
         return fail(c, RWNMR_ERR_INVALID, "set_unfolded: mode must be 0 .. 6");
     c->unfolded = enable;
     c->form_auto = false;
+    c->ran_shape.threads = 0;
     return RWNMR_OK;
 }
 
@@ -1352,6 +1371,7 @@ rwnmr_status rwnmr_ctx_set_launch(rwnmr_ctx *c, uint32_t tpb, uint32_t k)
     c->shape.threads = tpb;
     c->shape.k = k;
     c->shape_auto = use_default;
+    c->ran_shape.threads = 0;
     return RWNMR_OK;
 }
 
@@ -1359,8 +1379,9 @@ rwnmr_status rwnmr_ctx_get_launch(const rwnmr_ctx *c, uint32_t *tpb, uint32_t *k
 {
     if (!c || !tpb || !k)
         return RWNMR_ERR_INVALID;
-    *tpb = c->shape.threads;
-    *k = c->shape.k;
+    const LaunchShape ls = shape_in_use(c);
+    *tpb = ls.threads;
+    *k = ls.k;
     return RWNMR_OK;
 }
 
@@ -1764,12 +1785,13 @@ rwnmr_status rwnmr_ctx_get_tuning(const rwnmr_ctx *c, uint32_t *threads_per_bloc
 {
     if (!c)
         return RWNMR_ERR_INVALID;
+    const LaunchShape ls = shape_in_use(c);
     if (threads_per_block)
-        *threads_per_block = c->shape.threads;
+        *threads_per_block = ls.threads;
     if (walkers_per_lane)
-        *walkers_per_lane = c->shape.k;
+        *walkers_per_lane = ls.k;
     if (unfolded)
-        *unfolded = c->unfolded;
+        *unfolded = form_in_use(c);
     if (resort_every)
         *resort_every = c->resort_every;
     return RWNMR_OK;
@@ -1807,7 +1829,7 @@ rwnmr_status rwnmr_cpmg_run_noalloc(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_
     // 64-thread blocks have more echo partials: not where these would split the run
     if (shape.threads < c->shape.threads &&
         ((uint64_t)echoes + 1) * rwnmr::walk_grid_blocks(w->n, shape, (int)shift) > part_doubles)
-        shape = c->shape;
+        shape = c->ran_shape = c->shape;
     const uint32_t blocks = rwnmr::walk_grid_blocks(w->n, shape, (int)shift);
     // echoes per launch: rows 0..chunk of [echo][block] partials must fit the scratch
     uint64_t chunk = echoes ? echoes : 1;
@@ -1905,7 +1927,7 @@ rwnmr_status rwnmr_cpmg_graph_create(rwnmr_ctx *c, const rwnmr_image *img, rwnmr
     // 64-thread blocks have more echo partials: not where these would split the run
     if (shape.threads < c->shape.threads &&
         ((uint64_t)echoes + 1) * rwnmr::walk_grid_blocks(n, shape, 0) > kMaxPartialBytes / 8)
-        shape = c->shape;
+        shape = c->ran_shape = c->shape;
     const uint32_t blocks = rwnmr::walk_grid_blocks(n, shape, 0);
     uint64_t chunk = echoes ? echoes : 1;
     if (echo_sums && blocks)
