@@ -152,20 +152,23 @@ typedef struct {
 } rwnmr_walkers;
 
 /* Autotuner: times trial_echoes-long CPMG runs of copies of the walkers and
- * keeps the fastest settings in the context, in three steps: (1) the launch
+ * keeps the fastest settings in the context, in four steps: (1) the launch
  * shape, threads per block 64..1024 x walkers per lane 1/2/4 (walk kernel
  * time); (2) the image form the walk reads, the unfolded Z-order image with
  * the per-walker register chunk cache against the folded brick-ordered
- * bitBlock words (rwnmr_ctx_set_unfolded 3 / 0; walk kernel time), for
- * mirror walks the 8-byte chunk against the 16-byte one (6 / 3, each timed
- * twice in mirrored order), and for at most 65,536 walkers with one walker
- * per lane the speculative walk (5); (3) for
- * runs that use the locality ordering, the echoes per launch between walker
- * re-sorts, trial_echoes / 4, / 2 or trial_echoes (whole-run time, re-sorts
- * included).  best_* report step 1's shape and the fastest walk time; the
- * rest is read back with rwnmr_ctx_get_tuning.  The reference fixes all of
- * this in its config (BLOCKS/THREADSPERBLOCK/ECHOESPERKERNEL,
- * config/default/rwnmr.config:43-47). */
+ * bitBlock words (rwnmr_ctx_set_unfolded 3 / 0; walk kernel time), the
+ * 8-byte chunk against the 16-byte one where the walk has it (6 / 3, each
+ * timed twice in mirrored order), and for at most 65,536 walkers the
+ * speculative walk (5) in blocks of 64, of 256 and of step 1's threads; (3)
+ * what the context takes by itself, where no shape or no form was asked for:
+ * that stays, and stays automatic for runs of other sizes, unless the best so
+ * far is more than 1% faster; (4) for runs that use the locality ordering, the
+ * echoes per launch between walker re-sorts, trial_echoes / 4, / 2 or
+ * trial_echoes (whole-run time, re-sorts included).  best_* report the shape
+ * kept and its walk time; the rest is read back with rwnmr_ctx_get_tuning.
+ * Short runs stay unsorted unless rwnmr_ctx_set_locality was called.  The
+ * reference fixes all of this in its config
+ * (BLOCKS/THREADSPERBLOCK/ECHOESPERKERNEL, config/default/rwnmr.config:43-47). */
 rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *ctx, const rwnmr_image *img, const rwnmr_walkers *w,
                                 uint32_t steps_per_echo, int32_t bc, uint32_t trial_echoes,
                                 uint32_t *best_threads, uint32_t *best_k, double *best_ms);

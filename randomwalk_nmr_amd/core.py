@@ -103,7 +103,8 @@ class Context:
 
     def autotune(self, img, x, y, z, seed, *, steps_per_echo, bc="mirror", trial_echoes=64, penalty=None,
                  delta=1.0):
-        """Pick the fastest launch shape on copies of these walkers
+        """Pick the fastest launch shape and image form on copies of these
+        walkers, or leave both automatic where nothing is more than 1% faster
         (rwnmr_ctx_autotune).  Returns (threads_per_block, walkers_per_lane, ms)."""
         dev = _is_dev(x)
         if dev:

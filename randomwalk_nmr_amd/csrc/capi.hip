@@ -1592,7 +1592,11 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
     const int saved_unfolded = c->unfolded;
     const uint32_t saved_resort = c->resort_every;
     const bool saved_form_auto = c->form_auto, saved_shape_auto = c->shape_auto, saved_locality_auto = c->locality_auto;
+    const LaunchShape saved_ran = c->ran_shape;
+    const int saved_ran_form = c->ran_form;
     auto restore = [&]() {
+        c->ran_shape = saved_ran;
+        c->ran_form = saved_ran_form;
         c->form_auto = saved_form_auto;
         c->shape_auto = saved_shape_auto;
         c->locality_auto = saved_locality_auto;
@@ -1605,7 +1609,8 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
         cleanup();
     };
     c->timing = true;
-    // each trial runs the shape, form and ordering it is set to
+    // each trial runs the shape, form and ordering it is set to; all of them are
+    // sorted alike (or not at all), so the walk kernels' time compares them
     c->form_auto = c->shape_auto = c->locality_auto = false;
     (void)hipStreamSynchronize(c->stream);
     timing_collect(c);
@@ -1699,11 +1704,11 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
         }
         c->unfolded = best_form;
     }
-    // mirror walks: the 8-byte (4 x 4 x 4 voxel) chunk cache (form 6; 3 VALU
-    // per step fewer, a quarter more chunk loads) against the 16-byte one.
+    // the 8-byte (4 x 4 x 4 voxel) chunk cache (form 6; 3 VALU per step fewer, a
+    // quarter more chunk loads) against the 16-byte one, where the walk has it.
     // They differ by a few percent, so each is timed twice, in mirrored order,
     // and keeps its better time
-    if (bc == rwnmr::kMirror && best_form == 3 && saved_unfolded >= 3) {
+    if ((bc == rwnmr::kMirror || best.k == 1) && best_form == 3 && saved_unfolded >= 3) {
         double form_ms[2] = {1e300, 1e300};
         const int forms[2] = {3, 6};
         for (int t = 0; t < 4; ++t) {
@@ -1725,19 +1730,57 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
         c->unfolded = best_form;
     }
     // runs of at most one wave per SIMD are latency-bound: the speculative
-    // two-candidate walk (form 5, one walker per lane) against the rest
-    if (saved_unfolded >= 3 && c->shape.k == 1 && n <= kSpecMaxWalkers) {
-        c->unfolded = 5;
-        double ms = 0.0;
-        if ((s = trial(ms, false)) != RWNMR_OK) {
-            restore();
-            return s;
+    // two-candidate walk (form 5, one walker per lane) against the rest, in the
+    // block sizes it has its waves on most CUs with, whatever shape won above
+    if (saved_unfolded >= 3 && n <= kSpecMaxWalkers) {
+        const LaunchShape chunk_shape = best;
+        const bool third = chunk_shape.k == 1 && chunk_shape.threads != 64u && chunk_shape.threads != 256u;
+        const uint32_t spec_threads[3] = {64u, 256u, chunk_shape.threads};
+        for (int i = 0; i < (third ? 3 : 2); ++i) {
+            const uint32_t t = spec_threads[i];
+            c->shape = LaunchShape{t, 1u};
+            c->unfolded = 5;
+            double ms = 0.0;
+            if ((s = trial(ms, false)) != RWNMR_OK) {
+                restore();
+                return s;
+            }
+            if (ms < best_t) {
+                best_t = ms;
+                best_form = 5;
+                best = c->shape;
+            }
         }
-        if (ms < best_t) {
-            best_t = ms;
-            best_form = 5;
+    }
+    c->shape = best;
+    c->unfolded = best_form;
+    // what the context would take by itself, where the caller left that open:
+    // kept, and left automatic for runs of other sizes, unless the best is more
+    // than 1% faster
+    bool automatic = false;
+    if (saved_form_auto || saved_shape_auto) {
+        c->shape = saved;
+        c->unfolded = saved_unfolded;
+        c->form_auto = saved_form_auto;
+        c->shape_auto = saved_shape_auto;
+        double own = 1e300;
+        for (int t = 0; t < 2; ++t) {
+            double ms = 0.0;
+            if ((s = trial(ms, false)) != RWNMR_OK) {
+                restore();
+                return s;
+            }
+            own = std::min(own, ms);
         }
-        c->unfolded = best_form;
+        automatic = own <= 1.01 * best_t;
+        if (automatic) {
+            best_t = own;
+            best = shape_in_use(c);
+        } else {
+            c->shape = best;
+            c->unfolded = best_form;
+            c->form_auto = c->shape_auto = false;
+        }
     }
     // 3. echoes per launch of locality-ordered runs (the re-sort interval),
     // timed over the whole run with its re-sorts; the candidates differ by
@@ -1767,9 +1810,14 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *c, const rwnmr_image *img, const rwnm
     c->timing = was_timing;
     c->kernel_ms = saved_ms;
     c->kernel_launches = saved_launches;
-    c->shape = best;
-    c->unfolded = best_form;
+    if (!automatic) {
+        c->shape = best;
+        c->unfolded = best_form;
+    }
     c->resort_every = best_resort;
+    // the trials are cut from long runs and were sorted as these are: short
+    // runs stay unsorted unless the caller asked otherwise
+    c->locality_auto = saved_locality_auto;
     cleanup();
     if (best_threads)
         *best_threads = best.threads;

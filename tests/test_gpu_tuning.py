@@ -65,3 +65,41 @@ def test_read_back_of_settings():
         ctx.set_launch(0, 0)
         assert ctx.get_launch() == (256, 1)
         img.close()
+
+
+@pytest.mark.parametrize("bc", ["noflux", "periodic", "mirror"])
+@pytest.mark.parametrize("n", [3000, 70_000])
+def test_tuned_context_walks_runs_of_other_sizes(bc, n):
+    """Tuned for n walkers, then runs of n, of few and of many: as a context
+    left alone.  Short runs of many walkers are not sorted by the tuning."""
+    print(f"[test] tuned, other sizes bc={bc} n={n}", flush=True)
+    solid, *w = _inputs((48, 40, 32), 90_000, 5)
+    kw = dict(echoes=6, steps_per_echo=5, bc=bc, delta=0.995)
+    out = []
+    for tuned in (False, True):
+        with R.Context(0) as ctx:
+            img = R.Image.from_solid(ctx, solid)
+            if tuned:
+                tpb, k, ms = ctx.autotune(img, *(a[:n] for a in w), steps_per_echo=5, bc=bc, trial_echoes=30,
+                                          delta=0.995)
+                t = ctx.get_tuning()
+                assert t[:2] == (tpb, k) and ms > 0
+                # every form that the library takes by itself here is a candidate
+                assert t[2] in ((0, 3, 5, 6) if n <= 65_536 else (0, 3, 6))
+            out.append([R.cpmg_run(ctx, img, *(a[:m] for a in w), **kw) for m in (n, 500, 90_000)])
+            img.close()
+    for g, o in zip(out[1], out[0]):
+        _same(g, o)
+
+
+def test_tuning_keeps_what_was_asked_for():
+    """A form and a shape set by the caller leave nothing automatic to return to."""
+    print("[test] tuned, form and shape set", flush=True)
+    solid, *w = _inputs((32, 32, 32), 2000, 6)
+    with R.Context(0) as ctx:
+        img = R.Image.from_solid(ctx, solid)
+        ctx.set_unfolded(0)
+        ctx.set_launch(512, 1)
+        tpb, k, _ = ctx.autotune(img, *w, steps_per_echo=3, bc="mirror", trial_echoes=20, delta=0.995)
+        assert ctx.get_tuning()[:3] == (tpb, k, 0)
+        img.close()
