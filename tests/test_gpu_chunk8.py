@@ -42,11 +42,19 @@ def test_forms_match_oracle(bc, dims, form):
 
 
 @pytest.mark.parametrize("bc,n,steps", [("mirror", 65_537, 20), ("mirror", 70_001, 10_400), ("noflux", 400_001, 8),
-                                        ("periodic", 400_001, 8), ("mirror", 524_287, 60), ("mirror", 524_288, 60)])
+                                        ("periodic", 400_001, 8), ("mirror", 524_287, 60), ("mirror", 524_288, 60),
+                                        ("mirror", 70_001, 9_996), ("periodic", 70_001, 10_000),
+                                        ("mirror", 524_287, 5_000), ("mirror", 524_288, 5_000),
+                                        ("mirror", 600_001, 4_400)])
 def test_unconfigured_runs_match_named_forms(bc, n, steps):
-    """Both sides of each line of the default choice against form 3, unsorted."""
+    """Default choices against form 3, unsorted: above the speculative walk, both
+    sides of the line from which runs are sorted (10,000 steps of up to 250,000
+    walkers, 2 ms of more), and sorted runs below, at and above the 1024-thread
+    blocks of 524,288 walkers, with tiles of whole blocks and balanced ones.
+    The unsorted lines of larger images follow below."""
     print(f"[test] default choice bc={bc} n={n} steps={steps}", flush=True)
-    solid, seeds, x, y, z, pen = _inputs((40, 32, 24), n, 9)
+    # balanced tiles need periods of 128 and more
+    solid, seeds, x, y, z, pen = _inputs((72, 64, 64) if n > 600_000 else (40, 32, 24), n, 9)
     out = []
     for asked in (False, True):
         with R.Context(0) as ctx:
