@@ -98,7 +98,7 @@ rwnmr_status rwnmr_ctx_set_locality(rwnmr_ctx *ctx, int32_t enable, uint32_t res
  * 2: unfolded, each walker also keeping the 16-byte chunk (8 x 4 x 4
  * voxels) of its last lookup in registers so most steps read no memory;
  * 3 and 4: the chunk tested by one shift and the next direction
- * drawn a step ahead, through the 4 KiB byte-key table (3) or the 64 KiB
+ * drawn a step ahead, through the 7.25 KiB byte-key table (3) or the 64 KiB
  * wide direction table (4).  Modes 3 and 4 also run noflux walks (image
  * sides >= 2) on the periodic unfolded image, and start mirror CPMG / map
  * walkers at their folded positions with reflection flags (mirrored

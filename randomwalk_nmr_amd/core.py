@@ -84,7 +84,7 @@ class Context:
         of sides >= 2, on the periodic unfolded image): 0 folded kernels, 1 unfolded image (no
         per-step fold), 2 unfolded + per-walker 16-byte chunk cache, 3 and 4
         the chunk tested by one shift and the next direction drawn a step
-        ahead, through the 4 KiB byte-key table (3) or the 64 KiB
+        ahead, through the 7.25 KiB byte-key table (3) or the 64 KiB
         wide direction table (4); 5 as 3, with CPMG and map walks of one walker per lane
         loading both possible next chunks a step ahead (latency-bound runs
         of few walkers); 6 as 3, with an 8-byte (4 x 4 x 4 voxel) chunk

@@ -213,10 +213,10 @@ struct rwnmr_ctx {
     // periodic / mirror walks on the unfolded image (built per image on first use):
     // 0 folded kernels, 1 unfolded, 2 unfolded with the per-walker 128-bit
     // chunk cache, 3 and 4 with the chunk tested by one shift and the next
-    // direction drawn a step ahead, through the 4 KiB byte-key table (3, the
-    // default) or the 64 KiB wide direction table (4); 5 the speculative
-    // CPMG and map walk; 6 as 3 with an 8-byte (4 x 4 x 4 voxel) chunk for
-    // mirror walks (others run 3)
+    // direction drawn a step ahead, through the 7.25 KiB byte-key table (3) or
+    // the 64 KiB wide direction table (4); 5 the speculative CPMG and map walk;
+    // 6 as 3 with an 8-byte (4 x 4 x 4 voxel) chunk for walks of one walker per
+    // lane and mirror walks.  With form_auto, 3 stands for 5, 6 or 3 by the run
     int unfolded = 3;
     // resident 1024-thread blocks of the flag-keyed mirror walk (two per CU):
     // the tile count of balanced tiles (zbalanced_tile_walkers)
@@ -666,10 +666,10 @@ constexpr uint64_t kSpecMaxWalkers = 1024ull * 64ull, kSpecMaxMapWalkers = 768ul
 
 // Use the unfolded-image kernel for this walk when one applies.  noflux_ok:
 // the caller's kernel also runs noflux walks on the periodic unfolded image
-// (the CPMG, map and PFGSE walks, with the pipelined forms 3 and 4 and every
+// (the CPMG, map and PFGSE walks, with the pipelined forms 3 and up and every
 // image size >= 2).  mflags_ok: the caller's kernel starts mirror walkers in
 // the first octant of the mirror image with reflection flags (the CPMG and
-// map walks, forms 3 and 4, both then on the byte-key table), so each launch
+// map walks, forms 3 and up, all then on the byte-key table), so each launch
 // begins with the walkers' image lines inside one eighth of the mirror
 // image.
 // build: false uses an unfolded image only when an earlier call built it
@@ -1168,7 +1168,8 @@ rwnmr_status cpmg_common(rwnmr_ctx *c, const rwnmr_image *img, rwnmr_walkers *w,
         timing_end(c, t0);
         if (echo_sums) {
             // rows 0..ne of this launch are echoes done..done+ne (row 0 repeats
-            // the previous launch's last echo with identical bits)
+            // the previous launch's last echo: the same bits, or where the
+            // walkers were ordered anew the same values in another order)
             RW_HIP(c, rwnmr::launch_reduce_rows(a.partials, (uint64_t)ne + 1, blocks, sums + done, c->stream));
         }
         if (jac && ne == echoes)

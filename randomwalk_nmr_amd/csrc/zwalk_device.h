@@ -206,7 +206,7 @@ __device__ __forceinline__ void zbuild_table_noflux(const ZLayout &zl, uint4 *ta
 // the wide table (zbuild_table_wide); 2: the 6-entry table reached through
 // the byte-key table `keys` (zbuild_key_table); 3: the 12-entry table of
 // zbuild_table_flipped reached through the flag-keyed tables `keys`
-// (zbuild_flag_key_table), fo = flags x 4096.
+// (zbuild_flag_key_table), fo = flags x kZKeyEntries.
 struct ZEntry {
     uint32_t m, add, dp, fx, fy;      // axis mask, dilated addend, packed displacement, wrap fix-up
     uint32_t mf, tgt, add2;           // noflux: face test and the turned-around addend (ZFace)
@@ -1022,7 +1022,7 @@ struct ZEchoRows {
 // to arrive.  The directions run ahead too: at step t the entry of step t + 2
 // is read from the table, through the key byte read a step earlier, and the
 // key of step t + 3 is drawn, so neither table read is waited for.  A step is
-// free of branches: a hit multiplies the energy by delta, a move by 1.0.
+// free of branches: the energy, the address and the displacement are selected.
 // Same walk, bit for bit, as zwalk_tile (EMODE 0 and 1; SUB as there).
 template <int EMODE, bool WRAPFIX, bool NOFLUX, bool MFLAGS, bool SUB>
 __device__ __forceinline__ void zwalk_tile_spec(const WalkArgs &a, uint64_t tile, double *part, uint64_t part_stride,

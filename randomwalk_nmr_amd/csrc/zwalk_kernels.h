@@ -18,8 +18,16 @@ static constexpr uint32_t kZFlush = 511;
 // zflush_interval steps.  A walker moves at most that many voxels per axis
 // between two flushes, less than half of every period, so the coordinate
 // change modulo the period is the move itself.  A flush costs about 70
-// instructions, a packed displacement 2 per step, so it pays from periods of
-// 128 (63 steps) on.
+// instructions, a packed displacement 2 per step, so by instructions alone the
+// line would lie at periods near 72.  Measured (16-byte chunk, ns per step,
+// address against packed displacement):
+//   CPMG, whose displacement is kept in a branch, up to kZMaskWalkers: shortest
+//   period 128, 100k walkers 230 and 257, 200k 302 and 308; 96, 100k 234 and
+//   256, 200k 307 both; 64, 100k 213 and 224, 200k 280 and 271.
+//   Maps, whose displacement costs an add and a select: 128, 100k 188 and 183,
+//   300k 303 and 311; 95, 300k 302 and 295.
+// So at 128 it pays at every walker count but the smallest maps, below only for
+// some.
 static constexpr uint32_t kZMinDispPeriod = 128;
 
 __host__ __device__ inline uint32_t zmin_period(const ZLayout &zl)
@@ -131,7 +139,8 @@ hipError_t launch_zkeys(const int32_t *x, const int32_t *y, const int32_t *z, ui
 hipError_t launch_zpfgse(const WalkArgs &a, const PfgseArgs &p, hipStream_t st);
 
 // CPMG (emode 1), map (emode 0) or per-label CPMG (emode 2, needs a.zlabels
-// and a.label_delta) walk on a.zwords / a.zl; a.shift must be 0.
+// and a.label_delta) walk on a.zwords / a.zl, which addresses sub-voxels where
+// a.shift is not 0 (voxel division; form 3 and up).
 hipError_t launch_zwalk(const WalkArgs &a, int emode, const LaunchShape &ls, hipStream_t st);
 
 // Label-set CPMG walk (a.n_label_sets <= 8 rows of a.n_labels deltas in
