@@ -210,8 +210,6 @@ def main():
         tpb, k, ms = ctx.autotune(img, X0, Y0, Z0, SEED0, steps_per_echo=spe, bc=args.bc, trial_echoes=1000,
                                   delta=delta)
         log(f"autotune: threads {tpb} x walkers/lane {k} ({ms:.2f} ms per 1000 echoes) in {time.time() - t:.1f}s")
-    tpb, k, form, resort = ctx.get_tuning()
-    log(f"tuning: {tpb} x {k}, image form {form}, re-sort every {resort} echoes")
 
     def one_step():
         X.copy_(X0)
@@ -246,6 +244,9 @@ def main():
         log(f"GFX clock not sampled ({sampler.error or 'no samples'})")
     kern_ms, launches = ctx.get_timing(reset=True)
     ctx.set_timing(False)
+    # what the runs took, also where shape and form are automatic
+    tpb, k, form, resort = ctx.get_tuning()
+    log(f"tuning: {tpb} x {k}, image form {form}, re-sort every {resort} echoes")
 
     walker_steps = float(N) * spe * E
     ms_per_step = (t1 - t0) * 1e3 / args.steps
@@ -472,16 +473,14 @@ def wl_small(args):
     elif not args.no_autotune:
         tpb, k, ms = ctx.autotune(img, X0, Y0, Z0, S0, steps_per_echo=spe, bc="mirror", trial_echoes=E, delta=delta)
         log(f"autotune: threads {tpb} x walkers/lane {k} ({ms:.3f} ms per {E} echoes)")
-    tpb, k = ctx.get_launch()
-    form = ctx.get_tuning()[2]
-    log(f"image form {form}")
-
     def run():
         X.copy_(X0), Y.copy_(Y0), Z.copy_(Z0), SD.copy_(S0), EN.fill_(1.0)
         R.cpmg_run(ctx, img, X, Y, Z, SD, echoes=E, steps_per_echo=spe, bc="mirror", delta=delta, energy=EN,
                    echo_sums=SUMS, sync=True)
     run()
     sec = _timed(run, 10)
+    tpb, k, form, _ = ctx.get_tuning()   # what the runs took
+    log(f"launch {tpb} x {k}, image form {form}")
     steps = float(N) * spe * E
     eager_sums = SUMS.cpu().numpy().copy()
     # the same run captured as a HIP graph (walker resets, walk, echo reduction) and replayed
