@@ -109,9 +109,8 @@ rwnmr_status rwnmr_ctx_set_locality(rwnmr_ctx *ctx, int32_t enable, uint32_t res
  * an 8-byte chunk (4 x 4 x 4 voxels: 3 VALU per step fewer, a quarter more
  * chunk loads) in walks of one walker per lane and mirror walks.  Until this
  * is called, CPMG runs of up to 65,536 and map runs of up to 49,152 walkers
- * take 5 (unless set_launch asked for more than 256 threads, 64 for a map, or
- * more than one walker per lane), and larger ones 6 or 3 by size.  Modes 3 and
- * up also walk divided images (shift > 0).  Walkers are identical in every
+ * take 5 (unless set_launch was called), and larger ones 6 or 3 by size.  Modes
+ * 3 and up also walk divided images (shift > 0).  Walkers are identical in every
  * mode, echo sums to rounding. */
 rwnmr_status rwnmr_ctx_set_unfolded(rwnmr_ctx *ctx, int32_t mode);
 
@@ -175,7 +174,8 @@ rwnmr_status rwnmr_ctx_autotune(rwnmr_ctx *ctx, const rwnmr_image *img, const rw
 /* The context's launch shape, image form (rwnmr_ctx_set_unfolded mode) and
  * echoes between locality re-sorts: shape and form as set, or where they are
  * automatic as the last CPMG or map run took them (256 x 1 and 3 before the
- * first).  Setting what was read back repeats that run's choice.
+ * first).  Setting both as read back repeats that run's choice (a shape
+ * alone also settles that a small run takes the chunk cache).
  * rwnmr_ctx_get_launch reports the same shape. */
 rwnmr_status rwnmr_ctx_get_tuning(const rwnmr_ctx *ctx, uint32_t *threads_per_block, uint32_t *walkers_per_lane,
                                   int32_t *unfolded, uint32_t *resort_every);

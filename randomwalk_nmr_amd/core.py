@@ -89,7 +89,7 @@ class Context:
         loading both possible next chunks a step ahead (latency-bound runs
         of few walkers); 6 as 3, with an 8-byte (4 x 4 x 4 voxel) chunk
         (3 VALU per step fewer, a quarter more chunk loads).  Until this is
-        called the run's size chooses 5, 6 or 3."""
+        called the run's size chooses 5 (unless set_launch was called), 6 or 3."""
         check(load().rwnmr_ctx_set_unfolded(self.handle, int(mode)), self.handle)
 
     def set_timing(self, enable: bool = True):

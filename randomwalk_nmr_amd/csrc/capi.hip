@@ -708,12 +708,9 @@ void attach_zimage(rwnmr_ctx *c, const rwnmr_image *img, int bc, int emode, Walk
         a.zwords = z->words;
         a.zl = z->zl;
         a.zcache = c->unfolded >= 2 ? (uint32_t)(c->unfolded - 1) : 0u;
-        // few walkers: the speculative walk, unless a form was asked for or a
-        // shape in which it loses to the chunk cache (8k to 65,536 walkers on
-        // 32^3 to 256^3, 256 threads: CPMG 0.75-1.02 of the chunk walk's time,
-        // maps up to 1.15 of it; 64 threads: 0.65-0.9 of it, both)
-        const bool spec_shape = c->shape_auto || (c->shape.k == 1 && c->shape.threads <= (emode == 0 ? 64u : 256u));
-        if (c->form_auto && spec_shape && emode < 2 &&
+        // few walkers: the speculative walk, unless a form or a shape was asked for
+        // (echo sums of a shape asked for keep the bits of its block sums)
+        if (c->form_auto && c->shape_auto && emode < 2 &&
             a.n <= (emode == 0 ? kSpecMaxMapWalkers : kSpecMaxWalkers))
             a.zcache = 4;
         a.zlabels = zlab;
