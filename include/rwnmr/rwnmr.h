@@ -64,8 +64,8 @@ rwnmr_status rwnmr_ctx_synchronize(rwnmr_ctx *ctx);
 void *rwnmr_ctx_stream(rwnmr_ctx *ctx);
 /* Launch shape for walk kernels: threads per block (64..1024, multiple of
  * 64) and walkers per lane (1, 2 or 4).  0 selects the built-in default: 256 x 1,
- * 64 x 1 for CPMG / map runs of up to 49,152 walkers, 1024 x 1 for sorted mirror
- * runs of 524,288 and more. */
+ * 64 x 1 for the speculative walk (CPMG runs of up to 65,536 and map runs of up to
+ * 49,152 walkers), 1024 x 1 for sorted mirror runs of 524,288 and more. */
 rwnmr_status rwnmr_ctx_set_launch(rwnmr_ctx *ctx, uint32_t threads_per_block, uint32_t walkers_per_lane);
 rwnmr_status rwnmr_ctx_get_launch(const rwnmr_ctx *ctx, uint32_t *threads_per_block, uint32_t *walkers_per_lane);
 /* HIP-event timing of every walk / PFGSE kernel launched on the context

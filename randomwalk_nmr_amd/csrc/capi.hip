@@ -655,7 +655,7 @@ const uint8_t *zlabels_for(rwnmr_ctx *c, const rwnmr_image *img, int bc)
 
 // Walker counts up to one wave per SIMD (1024 SIMDs x 64 lanes) take the
 // speculative walk (form 5), with its two loads per step: CPMG of 10k walkers
-// at 128^3 (mirror) 139 against 203 ns per step, of 65,536 191 against 196,
+// at 128^3 (mirror) 139 against 203 ns per step, of 65,536 185 against 196,
 // but 245 against 222 at 100k and 545 against 297 at 200k, where the loads of
 // several waves per SIMD queue up.  A map step waits for less, so there its
 // line lies where the last SIMD of a CU gets a wave: 49,152 walkers 138 against
@@ -795,10 +795,10 @@ uint64_t chunk8_walkers(uint64_t voxels, int emode)
 // Launch shape of a CPMG, map or per-label run (a as attach_zimage left it)
 // and, where no image form was asked for, the form of a chunk-cache walk.
 // `sorted`: the walkers are kept in position order.
-//  - The speculative walk runs in 64-thread blocks while it leaves a SIMD of
-//    each CU free, so that its waves spread over as many CUs as there are
-//    (128^3, 30k walkers: 152 ns per step against 176 with 256 threads;
-//    65,536 walkers: 178 against 167).
+//  - The speculative walk runs in 64-thread blocks, so that its waves spread
+//    over as many CUs as there are (128^3 mirror, 3 steps per echo, ns per step
+//    against 256 threads: 30k walkers 151 and 176, 53,000 165 and 177, 65,536 170
+//    and 178; 12 steps per echo 119 and 162, 160 and 163, 160 and 164).
 //  - The 8-byte chunk (form 6) saves 3 instructions per step and costs a
 //    quarter more chunk loads, which pays where these hit the L2: sorted runs
 //    whose part of the image that is read fits the 4 MiB of one XCD (256^3
@@ -814,7 +814,7 @@ LaunchShape plan_run(rwnmr_ctx *c, WalkArgs &a, int emode, bool sorted)
 {
     LaunchShape ls = c->shape;
     if (c->shape_auto && a.zwords && emode < 2) {
-        if (a.zcache == 4 && a.n <= kSpecMaxWalkers / 4 * 3)
+        if (a.zcache == 4 && a.n <= kSpecMaxWalkers)
             ls = LaunchShape{64u, 1u};
         else if (sorted && a.zmflags && a.n >= (uint64_t)c->balanced_slots * 1024u && c->balanced_slots)
             ls = LaunchShape{1024u, 1u};

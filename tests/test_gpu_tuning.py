@@ -26,7 +26,7 @@ def _same(g, o):
 
 
 # the lines of the automatic choice (sorted from about 2 ms of walk on)
-@pytest.mark.parametrize("n,spe,shape,form", [(2000, 3, (64, 1), 5), (49_152, 3, (64, 1), 5), (49_153, 3, (256, 1), 5),
+@pytest.mark.parametrize("n,spe,shape,form", [(2000, 3, (64, 1), 5), (49_152, 3, (64, 1), 5), (65_536, 3, (64, 1), 5),
                                               (65_537, 3, (256, 1), 6), (524_288, 1250, (1024, 1), 6)])
 def test_read_back_tells_what_ran_and_repeats_it(n, spe, shape, form):
     print(f"[test] read-back n={n} spe={spe}", flush=True)
